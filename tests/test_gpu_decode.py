@@ -228,3 +228,75 @@ def test_long_sequence_logits_match_oracle(hiplib, cfg, n):
         scale = float(np.abs(want).max())
         err = float(np.abs(got[pos] - want).max())
         assert err <= 1e-3 * scale + 1e-5, f"position {pos}: max abs error {err} (scale {scale})"
+
+
+def position_logits(cfg, weights, tokens):
+    """The oracle's logits after each token."""
+    kv = np.zeros(2 * cfg.n_layers * cfg.seq_len * cfg.kv_dim, np.float32)
+    return np.stack([oracle.llama_forward(cfg.as_dict(), weights, kv, int(tok), pos)
+                     for pos, tok in enumerate(tokens)])
+
+
+@pytest.mark.parametrize("cfg,n", [
+    # heads of 2, K of 16 and 48; the fewest positions that go together, a
+    # second tile of 16 with one position, and the whole cache
+    (LlamaConfig(dim=16, hidden_dim=48, n_layers=2, n_heads=8, n_kv_heads=4, vocab_size=34,
+                 seq_len=40), 4),
+    (LlamaConfig(dim=16, hidden_dim=48, n_layers=2, n_heads=8, n_kv_heads=4, vocab_size=34,
+                 seq_len=40), 17),
+    (LlamaConfig(dim=16, hidden_dim=48, n_layers=2, n_heads=8, n_kv_heads=4, vocab_size=34,
+                 seq_len=40), 40),
+    # heads of 16, a second pass of one position, 64 x 128 classifier tiles
+    # of which the last holds 6 rows
+    (LlamaConfig(dim=64, hidden_dim=160, n_layers=2, n_heads=4, n_kv_heads=2, vocab_size=16390,
+                 seq_len=300), 257),
+    # heads of 32 with three queries each; classifier tiles of 32 x 64 and 64 x 64
+    (LlamaConfig(dim=96, hidden_dim=112, n_layers=2, n_heads=3, n_kv_heads=1, vocab_size=4200,
+                 seq_len=260), 33),
+    (LlamaConfig(dim=96, hidden_dim=112, n_layers=2, n_heads=3, n_kv_heads=1, vocab_size=4200,
+                 seq_len=260), 200),
+    # heads of 256; heads of 128 and the widest rows of several stages
+    (LlamaConfig(dim=512, hidden_dim=256, n_layers=1, n_heads=2, n_kv_heads=1, vocab_size=256,
+                 seq_len=80), 65),
+    (LlamaConfig(dim=1024, hidden_dim=2816, n_layers=1, n_heads=8, n_kv_heads=8, vocab_size=384,
+                 seq_len=48), 16)])
+def test_given_positions_together_match_oracle(hiplib, cfg, n):
+    """Scored text and prompts whose positions go through the layers
+    together, at the edges of their tiles. The tolerance: f32 sums of up to
+    2816 terms in another order, sqrt(2816) 2^-24 = 3.2e-6 of their scale
+    each, four in a row per layer over two layers."""
+    announce(f"decode given positions {cfg} n={n}")
+    weights = make_model(cfg, seed=9)
+    tokens = list(make_prompt(cfg, n=n, seed=10))
+    want = position_logits(cfg, weights, tokens)
+    model = LlamaI8(hiplib, cfg, weights)
+    got = model.logits(tokens)
+    again = model.logits(tokens)
+    steps = min(6, cfg.seq_len - n + 1)
+    stream, gm = model.generate(tokens, steps)
+    model.close()
+    assert np.array_equal(got, again)
+    assert np.abs(got - want).max() <= 2.5e-5 * np.abs(want).max()
+    want_stream, margin = oracle.llama_generate(cfg.as_dict(), weights, tokens, steps)
+    assert_same_tokens(stream, want_stream, margin)
+    np.testing.assert_allclose(gm, margin, atol=1e-4)
+
+
+def test_later_positions_do_not_reach_earlier_ones(hiplib):
+    """A token whose embedding is infinite makes its own keys and values NaN:
+    the positions before it, in the same tile of 16, keep their logits."""
+    announce("decode given positions, one of them infinite")
+    cfg = LlamaConfig(dim=128, hidden_dim=256, n_layers=2, n_heads=2, n_kv_heads=1, vocab_size=64,
+                      seq_len=48)
+    weights = make_model(cfg, seed=9)
+    tokens = [t if t != 5 else 6 for t in map(int, make_prompt(cfg, n=24, seed=10))]
+    want = position_logits(cfg, weights, tokens[:21])
+    weights["tok_s"] = weights["tok_s"].copy()
+    weights["tok_s"][5] = np.inf
+    tokens[21] = 5
+    model = LlamaI8(hiplib, cfg, weights)
+    got = model.logits(tokens)
+    model.close()
+    rows = [r for r in range(cfg.vocab_size) if r != 5]  # the classifier shares the table
+    assert np.abs(got[:21, rows] - want[:, rows]).max() <= 2.5e-5 * np.abs(want).max()
+    assert np.isnan(got[21:, rows]).all()

@@ -5,18 +5,22 @@
  * Weights are re-laid out once at upload so each fused kernel streams one
  * matrix: per layer [Wq; Wk; Wv] stacked (one GEMV feeds RoPE and the KV
  * cache) and W1/W3 interleaved row by row (one GEMV feeds SwiGLU). The
- * position and the next token live in device memory; a step is a fixed
- * sequence of 5 * layers + 1 launches that, with VX_LLAMA_GRAPH, is captured
- * into hipGraphs of kGraphSteps steps and of one step (kept with the model
- * while the prompt length and I/O buffers stay the same) and replayed with
- * no host synchronisation until the tokens are read back.
+ * position and the next token live in device memory. Positions whose token is
+ * given (a prompt, a text to score) go through the layers together
+ * (kernels/prefill.hip); a step is a fixed sequence of 5 * layers + 1
+ * launches that, with VX_LLAMA_GRAPH, is captured into hipGraphs of
+ * kGraphSteps steps and of one step (kept with the model while the prompt
+ * length and I/O buffers stay the same) and replayed with no host
+ * synchronisation until the tokens are read back.
  */
 #include "../../include/vx_hardware_runtime.h"
 #include "../../include/vx_hip_ops.h"
 #include "vx_decode_kernels.h"
 #include "vx_hip_common.h"
+#include "vx_kernels.h"
 #include "vx_ops_internal.h"
 
+#include <algorithm>
 #include <cstring>
 #include <vector>
 
@@ -28,6 +32,10 @@ namespace {
 #define VX_DEC_GRAPH_STEPS 8
 #endif
 constexpr int kGraphSteps = VX_DEC_GRAPH_STEPS;
+/* Given positions from which they go together (prefill) rather than step by
+ * step: at the dim-768, 12-layer decoder a step takes 185 us, up to 16
+ * positions together with one classified 547 us. */
+constexpr int kPrefillMin = 4;
 
 struct LlamaI8 {
   vx_llama_i8_config cfg;
@@ -45,6 +53,11 @@ struct LlamaI8 {
   float *out_margin = nullptr;
   vxk::StepBest *best = nullptr; /* one per classifier workgroup */
   int prompt_cap = 0, out_cap = 0;
+  /* Given positions together: their residual stream and q, the GEMMs' input
+   * planes (dim and hidden wide), and (taken when logits are first asked
+   * for) their logits. */
+  float *px = nullptr, *pq = nullptr, *plogits = nullptr;
+  uint16_t *pdim = nullptr, *phid = nullptr;
   hipStream_t stream = nullptr;
   /* The instantiated step graphs (one step, kGraphSteps steps; [1]: for
    * steps whose positions are all below step_attention_near, whose
@@ -136,6 +149,22 @@ vxk::StepArgmaxArgs argmax_args(LlamaI8 &m, int n_prompt) {
   return a;
 }
 
+/* Final RMSNorm and classifier of the residual stream x: logits, the best
+ * candidates, and pos moved on by one. */
+void enqueue_classifier(LlamaI8 &m, const float *x) {
+  vxk::StepGemvArgs lg{};
+  lg.w = m.tok_q;
+  lg.scale = m.tok_s;
+  lg.rows = m.cfg.vocab_size;
+  lg.cols = m.cfg.dim;
+  lg.x = x;
+  lg.norm = m.rms_final;
+  lg.out = m.logits;
+  lg.pos = m.pos;
+  lg.part = m.best;
+  vxk::step_gemv_logits(lg, m.stream);
+}
+
 /* One token step on the model's stream; `near`: its position is below
  * step_attention_near (the attention launches take smaller rounds). */
 void enqueue_step(LlamaI8 &m, int n_prompt, bool near) {
@@ -213,17 +242,80 @@ void enqueue_step(LlamaI8 &m, int n_prompt, bool near) {
     w2.out = m.x;
     vxk::step_gemv_resid(w2, m.stream);
   }
-  vxk::StepGemvArgs lg{};
-  lg.w = m.tok_q;
-  lg.scale = m.tok_s;
-  lg.rows = c.vocab_size;
-  lg.cols = c.dim;
-  lg.x = m.x;
-  lg.norm = m.rms_final;
-  lg.out = m.logits;
-  lg.pos = m.pos;
-  lg.part = m.best;
-  vxk::step_gemv_logits(lg, m.stream);
+  enqueue_classifier(m, m.x);
+}
+
+/* Positions pos0 .. pos0 + count - 1 (count at most kPrefillCap) of the
+ * uploaded tokens through every layer together: their keys and values into
+ * the cache, the residual stream after the last layer in px. */
+void enqueue_prefill(LlamaI8 &m, int pos0, int count) {
+  const vx_llama_i8_config &c = m.cfg;
+  const int qkv_rows = c.dim + 2 * m.kv_dim;
+  const int64_t layer_kv = (int64_t)c.seq_len * m.kv_dim;
+  const int dim_kp = vxk::prefill_kp(c.dim), hid_kp = vxk::prefill_kp(c.hidden_dim);
+  vxk::prefill_embed_launch(m.prompt + pos0, m.tok_q, m.tok_s, m.px, count, c.dim, m.stream);
+  for (int l = 0; l < c.n_layers; ++l) {
+    vxk::PrefillGemmArgs g{};
+    g.count = count;
+    g.pos0 = pos0;
+    g.dim = c.dim;
+    g.kv_dim = m.kv_dim;
+    g.hs = m.hs;
+    g.cols = c.dim;
+    g.x = m.pdim;
+    g.kp = dim_kp;
+
+    vxk::prefill_norm_launch(m.px, m.rms_att + (int64_t)l * c.dim, m.pdim, count, c.dim, m.stream);
+    vxk::PrefillGemmArgs qkv = g;
+    qkv.w = m.wqkv + (int64_t)l * qkv_rows * c.dim;
+    qkv.scale = m.sqkv + (int64_t)l * qkv_rows;
+    qkv.rows = qkv_rows;
+    qkv.out = m.pq;
+    qkv.kcache = m.kcache + l * layer_kv;
+    qkv.vcache = m.vcache + l * layer_kv;
+    qkv.rope = m.rope;
+    vxk::prefill_qkv_launch(qkv, m.stream);
+
+    vxk::PrefillAttnArgs at;
+    at.q = m.pq;
+    at.kcache = qkv.kcache;
+    at.vcache = qkv.vcache;
+    at.planes = m.pdim;
+    at.kp = dim_kp;
+    at.count = count;
+    at.pos0 = pos0;
+    at.kv_dim = m.kv_dim;
+    at.hs = m.hs;
+    at.kv_mul = c.n_heads / c.n_kv_heads;
+    at.seq_len = c.seq_len;
+    vxk::prefill_attention_launch(at, c.n_heads, m.stream);
+
+    vxk::PrefillGemmArgs wo = g;
+    wo.w = m.wo + (int64_t)l * c.dim * c.dim;
+    wo.scale = m.so + (int64_t)l * c.dim;
+    wo.rows = c.dim;
+    wo.out = m.px;
+    vxk::prefill_resid_launch(wo, m.stream);
+
+    vxk::prefill_norm_launch(m.px, m.rms_ffn + (int64_t)l * c.dim, m.pdim, count, c.dim, m.stream);
+    vxk::PrefillGemmArgs ffn = g;
+    ffn.w = m.w13 + (int64_t)l * 2 * c.hidden_dim * c.dim;
+    ffn.scale = m.s13 + (int64_t)l * 2 * c.hidden_dim;
+    ffn.rows = 2 * c.hidden_dim;
+    ffn.planes = m.phid;
+    ffn.planes_kp = hid_kp;
+    vxk::prefill_swiglu_launch(ffn, m.stream);
+
+    vxk::PrefillGemmArgs w2 = g;
+    w2.w = m.w2 + (int64_t)l * c.dim * c.hidden_dim;
+    w2.scale = m.s2 + (int64_t)l * c.dim;
+    w2.rows = c.dim;
+    w2.cols = c.hidden_dim;
+    w2.x = m.phid;
+    w2.kp = hid_kp;
+    w2.out = m.px;
+    vxk::prefill_resid_launch(w2, m.stream);
+  }
 }
 
 } // namespace
@@ -331,6 +423,17 @@ void *vx_llama_i8_create(const vx_llama_i8_config *cfg,
   m->pos = alloc<int>(*m, 1);
   m->best = alloc<vxk::StepBest>(*m, (size_t)vxk::step_logits_groups(c.vocab_size));
   VX_HIP_CHECK(hipStreamCreateWithFlags(&m->stream, hipStreamNonBlocking));
+  if (c.seq_len >= kPrefillMin) {
+    /* one block: x and q, then the planes, whose columns past the width stay 0 */
+    const size_t cap = vxk::kPrefillCap;
+    const size_t pdim = (size_t)vxk::prefill_planes(c.dim);
+    const size_t phid = (size_t)vxk::prefill_planes(c.hidden_dim);
+    m->px = alloc<float>(*m, 2 * cap * D + (pdim + phid) / 2);
+    m->pq = m->px + cap * D;
+    m->pdim = reinterpret_cast<uint16_t *>(m->pq + cap * D);
+    m->phid = m->pdim + pdim;
+    VX_HIP_CHECK(hipMemsetAsync(m->pdim, 0, (pdim + phid) * sizeof(uint16_t), m->stream));
+  }
   return m;
 }
 
@@ -356,9 +459,20 @@ int32_t vx_llama_i8_generate(void *model, const int32_t *prompt,
   VX_HIP_CHECK(hipMemcpyAsync(m->prompt, prompt, sizeof(int) * n_prompt,
                               hipMemcpyHostToDevice, m->stream));
   vxk::StepArgmaxArgs start = argmax_args(*m, n_prompt);
-  vxk::step_start_launch(start, m->stream);
   const int positions = n_prompt + n_steps - 1;
   const int near_pos = vxk::step_attention_near(m->hs);
+  int p = 0; /* the first position that takes a step of its own */
+  if (n_prompt >= kPrefillMin) {
+    int count = 0;
+    for (; p < n_prompt; p += count) {
+      count = std::min(n_prompt - p, vxk::kPrefillCap);
+      enqueue_prefill(*m, p, count);
+    }
+    vxk::fill_i32_launch(m->pos, n_prompt - 1, m->stream);
+    enqueue_classifier(*m, m->px + (int64_t)(count - 1) * m->cfg.dim);
+  } else {
+    vxk::step_start_launch(start, m->stream);
+  }
   if (flags & VX_LLAMA_GRAPH) {
     if (m->step_exec_prompt != n_prompt) {
       drop_step_graph(*m);
@@ -381,7 +495,6 @@ int32_t vx_llama_i8_generate(void *model, const int32_t *prompt,
       }
       return exec;
     };
-    int p = 0;
     for (; kGraphSteps > 1 && p + kGraphSteps <= positions; p += kGraphSteps) {
       VX_HIP_CHECK(hipGraphLaunch(graph_for(p, kGraphSteps), m->stream));
     }
@@ -389,7 +502,7 @@ int32_t vx_llama_i8_generate(void *model, const int32_t *prompt,
       VX_HIP_CHECK(hipGraphLaunch(graph_for(p, 1), m->stream));
     }
   } else {
-    for (int p = 0; p < positions; ++p) {
+    for (; p < positions; ++p) {
       enqueue_step(*m, n_prompt, p < near_pos);
     }
   }
@@ -424,8 +537,34 @@ int32_t vx_llama_i8_logits(void *model, const int32_t *tokens, int32_t n,
   ensure_io(*m, n, 1);
   VX_HIP_CHECK(hipMemcpyAsync(m->prompt, tokens, sizeof(int) * n,
                               hipMemcpyHostToDevice, m->stream));
-  vxk::step_start_launch(argmax_args(*m, n), m->stream);
   const size_t vocab = (size_t)m->cfg.vocab_size;
+  if (n >= kPrefillMin) {
+    if (!m->plogits) {
+      m->plogits =
+          alloc<float>(*m, (size_t)std::min(vxk::kPrefillCap, m->cfg.seq_len) * vocab);
+    }
+    for (int p = 0; p < n; p += vxk::kPrefillCap) {
+      const int count = std::min(n - p, vxk::kPrefillCap);
+      enqueue_prefill(*m, p, count);
+      vxk::prefill_norm_launch(m->px, m->rms_final, m->pdim, count, m->cfg.dim, m->stream);
+      vxk::PrefillGemmArgs lg{};
+      lg.w = m->tok_q;
+      lg.scale = m->tok_s;
+      lg.rows = m->cfg.vocab_size;
+      lg.cols = m->cfg.dim;
+      lg.x = m->pdim;
+      lg.kp = vxk::prefill_kp(m->cfg.dim);
+      lg.count = count;
+      lg.out = m->plogits;
+      vxk::prefill_logits_launch(lg, m->stream);
+      VX_HIP_CHECK(hipGetLastError());
+      VX_HIP_CHECK(hipMemcpyAsync(logits + p * vocab, m->plogits, sizeof(float) * count * vocab,
+                                  hipMemcpyDeviceToHost, m->stream));
+    }
+    VX_HIP_CHECK(hipStreamSynchronize(m->stream));
+    return VX_OP_OK;
+  }
+  vxk::step_start_launch(argmax_args(*m, n), m->stream);
   const int near_pos = vxk::step_attention_near(m->hs);
   for (int p = 0; p < n; ++p) {
     enqueue_step(*m, n, p < near_pos);

@@ -34,6 +34,7 @@
 #include "../vx_hip_common.h"
 #include "../vx_kernels.h"
 #include "gemm_pp_layout.h"
+#include "vx_lds_dma.hip.h"
 
 #include <atomic>
 #include <map>
@@ -91,78 +92,8 @@ __device__ __forceinline__ void put(void *c, int64_t at, float v) {
  * offset past it reads zeros instead of faulting. */
 constexpr int kDStageK = pp::kStageK;
 constexpr int kDUnits = pp::kUnits; /* 16-byte units per plane */
-constexpr int kBufferFlags = 0x00020000;       /* raw 32-bit dwords */
 
 typedef short i16x4 __attribute__((ext_vector_type(4)));
-typedef int i32x4 __attribute__((ext_vector_type(4)));
-#define VX_LDS __attribute__((address_space(3)))
-
-/* Wait until at most `n` of this wave's vector memory operations are
- * outstanding (vmcnt n; lgkmcnt and expcnt untouched). */
-template <int n>
-__device__ __forceinline__ void wait_vm() {
-  static_assert(n >= 0 && n < 64, "vmcnt is 6 bits");
-  __builtin_amdgcn_s_waitcnt((n & 15) | ((n >> 4) << 14) | (7 << 4) | (15 << 8));
-}
-
-/* Wait until at most `newer` (0..kMax) whole stages of this wave's loads are
- * outstanding; each stage is kPer loads. */
-template <int kMax, int kPer>
-__device__ __forceinline__ void wait_stages(int newer) {
-  if constexpr (kMax >= 3) {
-    if (newer >= 3) {
-      wait_vm<3 * kPer>();
-      return;
-    }
-  }
-  if constexpr (kMax >= 2) {
-    if (newer >= 2) {
-      wait_vm<2 * kPer>();
-      return;
-    }
-  }
-  if constexpr (kMax >= 1) {
-    if (newer >= 1) {
-      wait_vm<kPer>();
-      return;
-    }
-  }
-  wait_vm<0>();
-}
-
-/* One 16-byte-per-lane load from the buffer `rsrc` at byte offset `voff`
- * into LDS at `lds` + 16*lane. Written as assembly so the compiler neither
- * waits for it at every LDS read (it cannot tell which ring slot the load
- * fills) nor drops the barrier-time vmcnt(0) it adds for a fenced barrier:
- * the kernel orders these loads itself with wait_vm and lds_barrier. The
- * nop covers the one wait state between the M0 write and its use. */
-#pragma clang diagnostic push
-#pragma clang diagnostic ignored "-Winline-asm" /* m0 is reserved: declared */
-__device__ __forceinline__ void dma16(i32x4 rsrc, uint32_t voff, uint32_t lds) {
-  asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tbuffer_load_dwordx4 %0, %1, 0 offen lds"
-               :
-               : "v"(voff), "s"(rsrc), "s"(lds)
-               : "memory", "m0");
-}
-#pragma clang diagnostic pop
-
-/* Workgroup barrier without the release fence __syncthreads carries (that
- * fence waits for every outstanding global load, the prefetches included).
- * LDS reads are drained first so a slot is never refilled under a reader. */
-__device__ __forceinline__ void lds_barrier() {
-  __builtin_amdgcn_s_waitcnt(0xc07f); /* lgkmcnt(0) */
-  asm volatile("s_barrier" ::: "memory");
-}
-
-__device__ __forceinline__ i32x4 buffer_rsrc(const void *base, int bytes) {
-  const uint64_t a = (uint64_t)base;
-  i32x4 r;
-  r[0] = (int)(uint32_t)a;
-  r[1] = (int)((uint32_t)(a >> 32) & 0xffffu); /* stride 0 */
-  r[2] = bytes;
-  r[3] = kBufferFlags;
-  return r;
-}
 
 /* Ping-pong variant on v_mfma_f32_16x16x32: the same 256x256 tile, the same
  * 4-slot ring of K=32 stages filled by buffer-to-LDS loads, 8 waves (2x4,

@@ -125,6 +125,51 @@ int step_attention_near(int hs);
 /* pos = 0. */
 void step_start_launch(const StepArgmaxArgs &a, hipStream_t s);
 
+/* ---- Given positions together (kernels/prefill.hip) ----
+ *
+ * A pass takes up to kPrefillCap positions. Activations that feed a GEMM are
+ * three bf16 planes [3][kPrefillCap][kp] whose sum is the f32 value; kp is the
+ * width rounded up to the widest stage of K, and columns from the width on
+ * must be zero. */
+constexpr int kPrefillCap = 256;
+constexpr int kPrefillMaxCols = 4096;
+inline int prefill_kp(int cols) { return (cols + 127) / 128 * 128; }
+inline int64_t prefill_planes(int cols) { return (int64_t)3 * kPrefillCap * prefill_kp(cols); }
+
+struct PrefillGemmArgs {
+  const int8_t *w;    /* [rows, cols] */
+  const float *scale; /* [rows] */
+  int rows, cols;     /* as step_gemv_ok */
+  const uint16_t *x;  /* planes of the input */
+  int kp;
+  int count;          /* positions, at most kPrefillCap */
+  int pos0;           /* the first one's place in the sequence */
+  float *out;         /* [count, dim] q, [count, rows] residual stream or logits */
+  uint16_t *planes;   /* SwiGLU's output */
+  int planes_kp;
+  float *kcache, *vcache; /* this layer's [seq, kv_dim] */
+  const float *rope;      /* [seq_len, hs / 2, 2] */
+  int dim, kv_dim, hs;
+};
+
+struct PrefillAttnArgs {
+  const float *q; /* [count, heads * hs] */
+  const float *kcache, *vcache;
+  uint16_t *planes;
+  int kp, count, pos0;
+  int kv_dim, hs, kv_mul, seq_len;
+};
+
+void prefill_embed_launch(const int *tokens, const int8_t *tok_q, const float *tok_s, float *x,
+                          int count, int dim, hipStream_t s);
+void prefill_norm_launch(const float *x, const float *w, uint16_t *planes, int count, int dim,
+                         hipStream_t s);
+void prefill_qkv_launch(const PrefillGemmArgs &a, hipStream_t s);
+void prefill_attention_launch(const PrefillAttnArgs &a, int heads, hipStream_t s);
+void prefill_resid_launch(const PrefillGemmArgs &a, hipStream_t s);
+void prefill_swiglu_launch(const PrefillGemmArgs &a, hipStream_t s);
+void prefill_logits_launch(const PrefillGemmArgs &a, hipStream_t s);
+
 } // namespace vxk
 
 #endif /* VX_AMD_DECODE_KERNELS_H */
