@@ -33,8 +33,10 @@
 #include "../../../include/vx_hardware_runtime.h"
 #include "../vx_hip_common.h"
 #include "../vx_kernels.h"
+#include "gemm_direct.h"
 #include "gemm_pp_layout.h"
 #include "vx_lds_dma.hip.h"
+#include "vx_mfma16.hip.h"
 
 #include <atomic>
 #include <map>
@@ -42,13 +44,14 @@
 #include <type_traits>
 
 namespace vxk {
+
+/* gemm_direct.hip */
+bool gemm_direct_takes(const GemmArgs &g);
+void gemm_direct_launch(const GemmArgs &g, const direct::Plan &plan, char *ws, hipStream_t s);
+
 namespace {
 
-typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
-typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
 typedef float f32x16 __attribute__((ext_vector_type(16)));
-typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
-typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
 
 constexpr int kTileM = pp::kTileM;
 constexpr int kTileN = pp::kTileN;
@@ -126,21 +129,6 @@ typedef short i16x4 __attribute__((ext_vector_type(4)));
  * transposing read touches land in distinct banks. Each accumulator adds its
  * 32-term stage sums in k order, so results are deterministic (not
  * bit-identical to the 32x32x16 kernels, which add 16-term sums). */
-
-typedef float f32x4 __attribute__((ext_vector_type(4)));
-
-template <bool kBf16>
-__device__ __forceinline__ f32x4 mfma16(u32x4 a, u32x4 b, f32x4 c) {
-  if constexpr (kBf16) {
-    return __builtin_amdgcn_mfma_f32_16x16x32_bf16(
-        __builtin_bit_cast(bf16x8, a), __builtin_bit_cast(bf16x8, b), c, 0, 0,
-        0);
-  } else {
-    return __builtin_amdgcn_mfma_f32_16x16x32_f16(
-        __builtin_bit_cast(f16x8, a), __builtin_bit_cast(f16x8, b), c, 0, 0,
-        0);
-  }
-}
 
 /* Four consecutive elements of C from `at` (one 16-byte store of f32, or
  * 8 bytes of bf16 / f16, where `vec` says the address allows it). */
@@ -1047,6 +1035,9 @@ struct SkSpace {
   char *base = nullptr;
   size_t bytes = 0;
   int seq = 0;
+  /* the register GEMM's split launches: tickets, then partial sums */
+  char *split = nullptr;
+  size_t split_bytes = 0;
 };
 std::mutex sk_mutex;
 std::atomic<int64_t> sk_launches{0};
@@ -1055,8 +1046,10 @@ std::map<std::pair<int, hipStream_t>, SkSpace> &sk_spaces() {
   return *m;
 }
 
-bool sk_reserve(SkSpace &sp, size_t bytes, hipStream_t stream) {
-  if (sp.base && bytes <= sp.bytes) {
+/* A block of at least `bytes` in `base`, its first `zeroed` bytes zero when it
+ * is fresh; false when there is none to be had. */
+bool sk_reserve(char *&base, size_t &held, size_t bytes, size_t zeroed, hipStream_t stream) {
+  if (base && bytes <= held) {
     return true;
   }
   void *fresh = nullptr;
@@ -1064,12 +1057,12 @@ bool sk_reserve(SkSpace &sp, size_t bytes, hipStream_t stream) {
     (void)hipGetLastError();
     return false;
   }
-  VX_HIP_CHECK(hipMemsetAsync(fresh, 0, (size_t)pp::kSkFlagBytes, stream));
-  if (sp.base) {
-    VX_HIP_CHECK(hipFreeAsync(sp.base, stream));
+  VX_HIP_CHECK(hipMemsetAsync(fresh, 0, zeroed, stream));
+  if (base) {
+    VX_HIP_CHECK(hipFreeAsync(base, stream));
   }
-  sp.base = static_cast<char *>(fresh);
-  sp.bytes = bytes;
+  base = static_cast<char *>(fresh);
+  held = bytes;
   return true;
 }
 
@@ -1106,7 +1099,8 @@ bool launch_sk_any(const GemmArgs &g, hipStream_t s) {
   const int64_t tiles = ((g.m + kTileM - 1) / kTileM) * ((g.n + kTileN - 1) / kTileN);
   const int cus = device_cu_count();
   const int id_base = pp::sk_base((int)tiles, cus, (int)(g.k / kDStageK));
-  if (!sk_reserve(sp, (size_t)pp::sk_bytes((int)(tiles - id_base - cus)), s)) {
+  if (!sk_reserve(sp.base, sp.bytes, (size_t)pp::sk_bytes((int)(tiles - id_base - cus)),
+                  (size_t)pp::kSkFlagBytes, s)) {
     return false;
   }
   sp.seq = sp.seq == INT32_MAX ? 1 : sp.seq + 1;
@@ -1121,6 +1115,41 @@ bool launch_sk_any(const GemmArgs &g, hipStream_t s) {
   }
   ++sk_launches;
   return true;
+}
+
+direct::Plan direct_plan(const GemmArgs &g, bool may_split, double *us) {
+  const bool odd = (g.lda & 1) || ((uintptr_t)g.a & 2);
+  return direct::plan(g.m, g.n, g.k, odd, device_cu_count(), may_split, us);
+}
+
+void launch_direct(const GemmArgs &g, hipStream_t s) {
+  double us;
+  direct::Plan plan = direct_plan(g, g.may_split, &us);
+  if (!plan.ws_bytes) {
+    gemm_direct_launch(g, plan, nullptr, s);
+    return;
+  }
+  std::lock_guard<std::mutex> hold(sk_mutex);
+  int dev = 0;
+  VX_HIP_CHECK(hipGetDevice(&dev));
+  SkSpace &sp = sk_spaces()[{dev, s}];
+  if (!sk_reserve(sp.split, sp.split_bytes, (size_t)plan.ws_bytes, (size_t)direct::kTicketBytes,
+                  s)) {
+    plan = direct_plan(g, false, &us);
+  }
+  gemm_direct_launch(g, plan, sp.split, s);
+}
+
+/* Microseconds of the ping-pong launches on a 256-CU MI355X: 9 and, a round
+ * of the CUs, 0.6 a stage of K while few CUs compute, up to 0.84 with all of
+ * them (4096^3 113 us, 64 x 4096 x 4096 81). The stream-K tail counts as the
+ * half round it is. */
+double pp_us(const GemmArgs &g) {
+  const double tiles = (double)(((g.m + kTileM - 1) / kTileM) * ((g.n + kTileN - 1) / kTileN));
+  const double cus = device_cu_count(), stages = (double)(g.k / kDStageK);
+  const double full = (double)(int64_t)(tiles / cus), part = tiles - full * cus;
+  const double tail = part == 0 ? 0.0 : full > 0 && part <= cus / 2 ? 0.5 : 1.0;
+  return 9.0 + stages * (0.6 + 0.24 * (full > 0 ? 1.0 : part / cus)) * (full + tail);
 }
 
 template <int kIn, int kOut>
@@ -1156,17 +1185,30 @@ bool gemm_kernel_takes(GemmKernel which, const GemmArgs &g) {
     return f32_mfma_takes(g);
   case GEMM_TILED:
     return tiled_takes(g);
+  case GEMM_MFMA_DIRECT:
+    return gemm_direct_takes(g);
   default:
     return false;
   }
 }
 
 GemmKernel gemm_pick(const GemmArgs &g) {
-  /* Small products stay on the exact-order kernel: a 256x256 tile of mostly
-   * padding costs more than it saves there. */
-  const bool big = g.m >= 64 && g.n >= 64 && (double)g.m * g.n * g.k >= 16777216.0;
-  if (big && pp_takes(g)) {
-    return sk_takes(g) ? GEMM_MFMA_SK : GEMM_MFMA_PP;
+  /* 16-bit products of 2^18 multiply-adds and K >= 128, or of 2^25: MFMA
+   * kernels (smaller ones stay exact-order: a launch is most of their time,
+   * 64^3 6.0 us). 256x256 tiles or the register GEMM, whichever takes less
+   * time by its model: 512 x 4096 x 4096 88 and 33 us, 4096^3 113 and 215. */
+  const double work = (double)g.m * (double)g.n * (double)g.k;
+  if (work >= 33554432.0 || (g.k >= 128 && work >= 262144.0)) {
+    double us = 1e30;
+    if (gemm_direct_takes(g)) {
+      (void)direct_plan(g, g.may_split, &us);
+    }
+    if (pp_takes(g) && pp_us(g) <= us) {
+      return sk_takes(g) ? GEMM_MFMA_SK : GEMM_MFMA_PP;
+    }
+    if (us < 1e30) {
+      return GEMM_MFMA_DIRECT;
+    }
   }
   /* f32: the exact-order kernel (bit-equal to the reference's host loop)
    * below 2^30 multiply-adds, the MFMA kernel above. */
@@ -1194,6 +1236,11 @@ bool gemm_launch_kernel(GemmKernel which, const GemmArgs &g,
     if (!launch_sk_any(g, stream)) {
       launch_pp_any(g, stream);
     }
+  } else if (which == GEMM_MFMA_DIRECT) {
+    if (!gemm_direct_takes(g)) {
+      return false;
+    }
+    launch_direct(g, stream);
   } else if (which == GEMM_F32_MFMA) {
     if (!f32_mfma_takes(g)) {
       return false;
@@ -1254,9 +1301,11 @@ int gemm_release_stream(hipStream_t stream) {
       ++it;
       continue;
     }
-    if (it->second.base) {
-      VX_HIP_CHECK(hipFreeAsync(it->second.base, stream));
-      ++freed;
+    for (char *p : {it->second.base, it->second.split}) {
+      if (p) {
+        VX_HIP_CHECK(hipFreeAsync(p, stream));
+        ++freed;
+      }
     }
     it = m.erase(it);
   }
@@ -1267,10 +1316,8 @@ void gemm_workspace_stats(int64_t *blocks, int64_t *bytes, int64_t *launches) {
   std::lock_guard<std::mutex> hold(sk_mutex);
   int64_t n = 0, total = 0;
   for (const auto &e : sk_spaces()) {
-    if (e.second.base) {
-      ++n;
-      total += (int64_t)e.second.bytes;
-    }
+    n += (e.second.base != nullptr) + (e.second.split != nullptr);
+    total += (int64_t)(e.second.bytes + e.second.split_bytes);
   }
   *blocks = n;
   *bytes = total;

@@ -26,17 +26,13 @@
 #include "../vx_hip_common.h"
 #include "../vx_decode_kernels.h"
 #include "vx_lds_dma.hip.h"
+#include "vx_mfma16.hip.h"
 #include "vx_wave_ops.hip.h"
 
 #include <cmath>
 
 namespace vxk {
 namespace {
-
-typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
-typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
-typedef float f32x4 __attribute__((ext_vector_type(4)));
-typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 
 constexpr int kThreads = 256;
 
@@ -143,11 +139,6 @@ __device__ __forceinline__ u32x4 widen(uint32_t lo, uint32_t hi) {
     }
   }
   return r;
-}
-
-__device__ __forceinline__ f32x4 mfma16(u32x4 a, u32x4 b, f32x4 c) {
-  return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, a),
-                                                 __builtin_bit_cast(bf16x8, b), c, 0, 0, 0);
 }
 
 enum PreMode { kPreQkv = 0, kPreResid = 1, kPreSwiglu = 2, kPreLogits = 3 };
@@ -317,9 +308,9 @@ __global__ __launch_bounds__(kThreads, 1) void prefill_gemm(PrefillGemmArgs a) {
           }
 #pragma unroll
           for (int i = 0; i < kRB; ++i) {
-            hi[i][j] = mfma16(wf[i][s], xf[0], hi[i][j]);
-            lo[i][j] = mfma16(wf[i][s], xf[1], lo[i][j]);
-            lo[i][j] = mfma16(wf[i][s], xf[2], lo[i][j]);
+            hi[i][j] = mfma16<true>(wf[i][s], xf[0], hi[i][j]);
+            lo[i][j] = mfma16<true>(wf[i][s], xf[1], lo[i][j]);
+            lo[i][j] = mfma16<true>(wf[i][s], xf[2], lo[i][j]);
           }
         }
       }

@@ -29,8 +29,8 @@ struct GemmArgs {
    * and real-time counter at the start and end of workgroup 0), or null. */
   uint64_t *stamp = nullptr;
   /* Whether the launch may take a workspace of its own (false under graph
-   * capture and for the no-alloc entry point): the stream-K launch needs
-   * one. */
+   * capture and for the no-alloc entry point): the stream-K launch and the
+   * register GEMM's splits need one. */
   bool may_split = false;
 };
 
@@ -44,10 +44,13 @@ enum GemmKernel {
   GEMM_MFMA_SK = 10, /* the ping-pong tiles on one workgroup per CU, the second
                         round's tiles cut at half of K between two workgroups
                         (grids of 1 to 1.5 rounds; needs a workspace) */
+  GEMM_MFMA_DIRECT = 11, /* bf16/f16 on 16x16x32 MFMAs fed from memory without
+                            LDS: any alignment, few rows, small grids */
 };
 
 inline bool gemm_is_mfma(GemmKernel k) {
-  return k == GEMM_MFMA_PP || k == GEMM_F32_MFMA || k == GEMM_MFMA_SK;
+  return k == GEMM_MFMA_PP || k == GEMM_F32_MFMA || k == GEMM_MFMA_SK ||
+         k == GEMM_MFMA_DIRECT;
 }
 
 GemmKernel gemm_pick(const GemmArgs &g);
@@ -59,10 +62,11 @@ bool gemm_launch(const GemmArgs &g, hipStream_t stream);
 bool gemm_launch_kernel(GemmKernel which, const GemmArgs &g,
                         hipStream_t stream);
 
-/* Frees, in `stream`'s order, the stream-K workspace kept for `stream` on
- * every device (none while it is capturing); the number freed. */
+/* Frees, in `stream`'s order, the workspaces (stream-K, the register GEMM's
+ * splits) kept for `stream` on every device (none while it is capturing); the
+ * number freed. */
 int gemm_release_stream(hipStream_t stream);
-/* Stream-K workspaces held, their bytes, and stream-K launches so far. */
+/* Workspaces held, their bytes, and stream-K launches so far. */
 void gemm_workspace_stats(int64_t *blocks, int64_t *bytes, int64_t *launches);
 
 /* *p = v on `stream` (one thread; a kernel rather than hipMemsetAsync so a

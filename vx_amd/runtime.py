@@ -139,8 +139,8 @@ class DispatchLibrary:
             raise ValueError(f"no GEMM kernel {which}")
 
     def gemm_workspaces(self) -> dict:
-        """Stream-K GEMM workspaces held (one per device and stream that ran
-        such a launch), their bytes, stream-K launches so far, and the
+        """GEMM workspaces held (one per device, stream and kind that ran there:
+        stream-K, the register GEMM's splits), their bytes, stream-K launches so far, and the
         workgroups (CUs) such a launch runs."""
         out = (ctypes.c_int64 * 4)()
         if not self.lib.vx_plugin_control(abi.HIP_CTRL_GEMM_WORKSPACES, out):
