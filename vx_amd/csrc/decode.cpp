@@ -422,7 +422,6 @@ void *vx_llama_i8_create(const vx_llama_i8_config *cfg,
   m->hb = alloc<float>(*m, H);
   m->pos = alloc<int>(*m, 1);
   m->best = alloc<vxk::StepBest>(*m, (size_t)vxk::step_logits_groups(c.vocab_size));
-  VX_HIP_CHECK(hipStreamCreateWithFlags(&m->stream, hipStreamNonBlocking));
   if (c.seq_len >= kPrefillMin) {
     /* one block: x and q, then the planes, whose columns past the width stay 0 */
     const size_t cap = vxk::kPrefillCap;
@@ -432,8 +431,12 @@ void *vx_llama_i8_create(const vx_llama_i8_config *cfg,
     m->pq = m->px + cap * D;
     m->pdim = reinterpret_cast<uint16_t *>(m->pq + cap * D);
     m->phid = m->pdim + pdim;
-    VX_HIP_CHECK(hipMemsetAsync(m->pdim, 0, (pdim + phid) * sizeof(uint16_t), m->stream));
+    VX_HIP_CHECK(hipMemset(m->pdim, 0, (pdim + phid) * sizeof(uint16_t)));
   }
+  /* the fills above are on the null stream, which the model's own does not
+   * wait for */
+  VX_HIP_CHECK(hipStreamSynchronize(nullptr));
+  VX_HIP_CHECK(hipStreamCreateWithFlags(&m->stream, hipStreamNonBlocking));
   return m;
 }
 
