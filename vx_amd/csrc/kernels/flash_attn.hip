@@ -43,6 +43,7 @@
  */
 #include "../vx_hip_common.h"
 #include "../vx_ops_kernels.h"
+#include "flash_rows.h"
 
 #include <algorithm>
 #include <atomic>
@@ -744,8 +745,11 @@ int pick_splits(int64_t items, int64_t key_blocks, int cus) {
  * the caller stream of a thread moves off it (flash_attn_release_stream);
  * the default stream's block lives until the process ends. */
 struct SplitSpace {
-  float *base = nullptr;
+  char *base = nullptr;
   size_t bytes = 0;
+  /* flash_rows: tickets, then partials */
+  char *rows = nullptr;
+  size_t rows_bytes = 0;
 };
 std::mutex spaces_mutex;
 std::map<std::pair<int, hipStream_t>, SplitSpace> &spaces() {
@@ -753,10 +757,10 @@ std::map<std::pair<int, hipStream_t>, SplitSpace> &spaces() {
   return *m;
 }
 
-/* Makes `sp` hold `bytes` on `stream` (caller holds spaces_mutex); false
- * when the memory cannot be had. */
-bool reserve(SplitSpace &sp, size_t bytes, hipStream_t stream) {
-  if (sp.base && bytes <= sp.bytes) {
+/* Makes `base` hold `bytes` on `stream`, the first `zeroed` of a fresh block
+ * zero (caller holds spaces_mutex); false when the memory cannot be had. */
+bool reserve(char *&base, size_t &held, size_t bytes, size_t zeroed, hipStream_t stream) {
+  if (base && bytes <= held) {
     return true;
   }
   void *fresh = nullptr;
@@ -764,12 +768,47 @@ bool reserve(SplitSpace &sp, size_t bytes, hipStream_t stream) {
     (void)hipGetLastError();
     return false;
   }
-  if (sp.base) {
-    VX_HIP_CHECK(hipFreeAsync(sp.base, stream));
+  if (zeroed) {
+    VX_HIP_CHECK(hipMemsetAsync(fresh, 0, zeroed, stream));
   }
-  sp.base = static_cast<float *>(fresh);
-  sp.bytes = bytes;
+  if (base) {
+    VX_HIP_CHECK(hipFreeAsync(base, stream));
+  }
+  base = static_cast<char *>(fresh);
+  held = bytes;
   return true;
+}
+
+/* Calls of up to kRowsMaxQ queries a head over at least kRowsMinK keys: all of
+ * a KV head's heads together (flash_rows.hip), where this kernel would give
+ * each head a workgroup of 128 rows. With 16 x 64 heads on 8, d 128, over 4096
+ * keys: 16 queries 308 -> 105 us, 32 queries 312 -> 208 (at 64 this kernel's
+ * rate, twice that of 32, is the higher). Over 31 keys its one launch of 24
+ * workgroups takes 5.5 us and flash_rows 6.3. */
+constexpr int kRowsMaxQ = 32;
+constexpr int kRowsMinK = 128;
+
+rows::Plan rows_plan(int64_t kv_total, int64_t rows, int64_t seq_k, int head_dim, int cus,
+                     bool allow_split) {
+  rows::Plan p{};
+  p.mt = rows <= 16 ? 1 : 2;
+  p.tiles = (int)((rows + 16 * p.mt - 1) / (16 * p.mt));
+  p.splits = 1;
+  const int64_t items = kv_total * p.tiles, blocks = (seq_k + 31) / 32;
+  if (allow_split && items <= rows::kMaxSplitItems) {
+    const int forced = forced_splits.load();
+    /* one workgroup per CU, two blocks of keys a wave, 16 partial results:
+     * 32 items over 4096 keys 16.4 us in 8 splits, 19.6 in 16; one item over
+     * 8192 keys 8.7 in 16, 9.4 in 32 */
+    const int64_t want =
+        forced > 0 ? std::min<int64_t>(forced, blocks) : std::min<int64_t>({cus / items, blocks / 8, 16});
+    p.splits = (int)std::max<int64_t>(1, want);
+  }
+  if (p.splits > 1) {
+    p.ws_bytes =
+        rows::kTicketBytes + items * p.splits * (int64_t)(16 * p.mt) * (head_dim + 2) * 4;
+  }
+  return p;
 }
 
 } // namespace
@@ -798,9 +837,11 @@ int flash_attn_release_stream(hipStream_t stream) {
       ++it;
       continue;
     }
-    if (it->second.base) {
-      VX_HIP_CHECK(hipFreeAsync(it->second.base, stream));
-      ++freed;
+    for (char *p : {it->second.base, it->second.rows}) {
+      if (p) {
+        VX_HIP_CHECK(hipFreeAsync(p, stream));
+        ++freed;
+      }
     }
     it = m.erase(it);
   }
@@ -811,10 +852,8 @@ void flash_attn_workspace_stats(int64_t *blocks, int64_t *bytes) {
   std::lock_guard<std::mutex> hold(spaces_mutex);
   int64_t n = 0, total = 0;
   for (const auto &e : spaces()) {
-    if (e.second.base) {
-      ++n;
-      total += (int64_t)e.second.bytes;
-    }
+    n += (e.second.base != nullptr) + (e.second.rows != nullptr);
+    total += (int64_t)(e.second.bytes + e.second.rows_bytes);
   }
   *blocks = n;
   *bytes = total;
@@ -844,6 +883,31 @@ bool flash_attn_fwd_launch(const uint16_t *q, const uint16_t *k,
   }
   const float scale_log2 = scale * 1.4426950408889634f;
   const int group = (int)(heads / kv_heads);
+  if (seq_q <= kRowsMaxQ && seq_k >= kRowsMinK) {
+    rows::Args a{q, k, v, o, lse, batch * kv_heads, group * (int)seq_q, (int)seq_q, (int)seq_k,
+                 scale_log2, causal};
+    rows::Plan plan = rows_plan(a.kv_total, a.rows, seq_k, (int)head_dim, device_cu_count(),
+                                allow_split);
+    if (a.kv_total * plan.tiles * plan.splits <= INT32_MAX) {
+      std::unique_lock<std::mutex> hold(spaces_mutex, std::defer_lock);
+      char *ws = nullptr;
+      if (plan.splits > 1) {
+        hold.lock(); /* through the launch, as below */
+        int dev = 0;
+        VX_HIP_CHECK(hipGetDevice(&dev));
+        SplitSpace &sp = spaces()[{dev, stream}];
+        if (reserve(sp.rows, sp.rows_bytes, (size_t)plan.ws_bytes, (size_t)rows::kTicketBytes,
+                    stream)) {
+          ws = sp.rows;
+        } else {
+          plan.splits = 1;
+        }
+      }
+      flash_rows_launch(a, plan, (int)head_dim, ws, stream);
+      VX_HIP_CHECK(hipGetLastError());
+      return true;
+    }
+  }
   constexpr int kBlockQ = 4 * 32 * VX_FA_QT;
   const int64_t items = bh * ((seq_q + kBlockQ - 1) / kBlockQ);
   const int64_t key_blocks = (seq_k + VX_FA_BK - 1) / VX_FA_BK;
@@ -862,8 +926,8 @@ bool flash_attn_fwd_launch(const uint16_t *q, const uint16_t *k,
     const size_t rows = (size_t)bh * (size_t)seq_q;
     const size_t bytes =
         (size_t)splits * rows * ((size_t)head_dim + 1) * sizeof(float);
-    if (reserve(sp, bytes, stream)) {
-      float *opart = sp.base;
+    if (reserve(sp.base, sp.bytes, bytes, 0, stream)) {
+      float *opart = reinterpret_cast<float *>(sp.base);
       float *lpart = opart + (size_t)splits * rows * (size_t)head_dim;
       if (head_dim == 128) {
         launch<128, VX_FA_QT, VX_FA_BK>(q, k, v, o, lse, (int)heads, group,
