@@ -17,14 +17,17 @@
  * them between the MFMAs of the stage before, and writes each plane's 16
  * bytes as the MFMA operands want them: [row][chunk of 8 k], chunks XORed so
  * that 16 rows at one chunk lie in distinct banks, for the reads and both
- * writes. What bounds it is the LDS: 192 KiB pass through it per stage, 1.25
- * us where few tiles run, against 0.7 for the MFMAs (taking the waves of a
- * SIMD in turns, reads against MFMAs, costs a barrier more and gave 126 us at
- * 2048^3).
+ * writes; three stages' loads are in flight (with two: 1999 x 2001 x 2003 107
+ * us against 98, 300 x 4000 x 4096 163 against 150). What bounds it: at 2048^3
+ * the matrix cores work 45% of the cycles, at 2.1 GHz under their load; a
+ * stage's operand reads (144 KiB) and its MFMAs follow one another between
+ * barriers (taking a SIMD's two waves in turns, one reading while the other
+ * multiplies, costs a barrier more and gave the same: 108 us).
  *
- * Against f32 MFMAs in the same tile: 2048^3 248 -> 113 us (152 TFLOP/s),
- * 1024^3 125 -> 46, 128 x 4096 x 4096 454 -> 156; error against 64 bits 8.1e-7
- * -> 2.5e-7 at 2048^3, 1.1e-6 -> 3.8e-7 at K = 4096.
+ * Against f32 MFMAs in the same tile: 2048^3 248 -> 92 us with new inputs each
+ * pass (188 TFLOP/s), 258 -> 106 with the same ones, 1024^3 125 -> 45, 128 x
+ * 4096 x 4096 454 -> 142; error against 64 bits 8.1e-7 -> 2.5e-7 at 2048^3,
+ * 1.1e-6 -> 3.8e-7 at K = 4096.
  */
 #include "../vx_hip_common.h"
 #include "../vx_kernels.h"
@@ -52,7 +55,7 @@ struct Regs {
   float a[8], b[8];
 };
 
-__device__ __forceinline__ int unit(int row, int c) { return row * 4 + (c ^ ((row >> 2) & 3)); }
+__device__ __forceinline__ int unit(int row, int c) { return row * 4 + (c ^ ((row >> 1) & 3)); }
 
 /* Eight values as the three planes' 16 bytes. */
 __device__ __forceinline__ void split8(const float (&x)[8], u32x4 (&p)[3]) {
@@ -190,17 +193,21 @@ __global__ __launch_bounds__(kThreads, 2) void gemm_f32_mfma(
       load_last(r, st);
     }
   };
-  Regs r0, r1;
-  load_any(r0, 0);
-  stash(r0, 0);
+  /* Entering stage s: it is in slot s % 2, the next in r[(s + 1) % 3], the one
+   * after in r[(s + 2) % 3]. */
+  Regs r[3];
+  load_any(r[0], 0);
   if (stages > 1) {
-    load_any(r0, 1);
+    load_any(r[1], 1);
   }
+  if (stages > 2) {
+    load_any(r[2], 2);
+  }
+  stash(r[0], 0);
   lds_barrier();
   int64_t st = 0;
-  /* Entering stage st: it is in slot st % 2, stage st + 1 in r0. */
   auto stage = [&](int64_t s, int slot, const Regs &next, Regs &after) {
-    load(after, s + 2);
+    load(after, s + 3);
     fragments(slot);
     multiply();
     stash(next, slot ^ 1);
@@ -211,18 +218,21 @@ __global__ __launch_bounds__(kThreads, 2) void gemm_f32_mfma(
     }
     lds_barrier();
   };
-  for (; st + 3 < whole; st += 2) {
-    stage(st, 0, r0, r1);
-    stage(st + 1, 1, r1, r0);
+  for (; st + 8 < whole; st += 6) {
+#pragma unroll
+    for (int i = 0; i < 6; ++i) {
+      stage(st + i, i & 1, r[(i + 1) % 3], r[i % 3]);
+    }
   }
   for (; st < stages; ++st) {
     const int slot = (int)(st & 1);
     fragments(slot);
     if (st + 1 < stages) {
-      stash(r0, slot ^ 1);
+      stash(r[1], slot ^ 1);
     }
-    if (st + 2 < stages) {
-      load_any(r0, st + 2);
+    r[1] = r[2];
+    if (st + 3 < stages) {
+      load_any(r[2], st + 3);
     }
     multiply();
     lds_barrier();
