@@ -52,7 +52,7 @@ HIP_CTRL_GEMM_WORKSPACES = CTRL_VENDOR_BASE + 10
 GEMV_AUTO, GEMV_ROWS, GEMV_DOT2_B4, GEMV_LDS = 0, 1, 2, 3
 # Kernels the GEMM control opcode can force (0 = automatic choice).
 GEMM_AUTO, GEMM_TILED, GEMM_MFMA_PP, GEMM_F32_MFMA, GEMM_MFMA_SK = 0, 2, 8, 9, 10
-GEMM_MFMA_DIRECT = 11
+GEMM_MFMA_DIRECT, GEMM_MFMA_RING = 11, 12
 
 
 def memref_tag(dtype: int, rank: int) -> int:

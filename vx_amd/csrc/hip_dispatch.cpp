@@ -1400,7 +1400,8 @@ int32_t vx_plugin_control(uint32_t opcode, void *payload) {
     const int32_t *which = static_cast<const int32_t *>(payload);
     if (!which || !(*which == 0 || *which == vxk::GEMM_TILED ||
                     *which == vxk::GEMM_MFMA_PP || *which == vxk::GEMM_F32_MFMA ||
-                    *which == vxk::GEMM_MFMA_SK || *which == vxk::GEMM_MFMA_DIRECT)) {
+                    *which == vxk::GEMM_MFMA_SK || *which == vxk::GEMM_MFMA_DIRECT ||
+                    *which == vxk::GEMM_MFMA_RING)) {
       return 0;
     }
     forced_gemm_kernel.store(*which);

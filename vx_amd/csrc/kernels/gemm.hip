@@ -36,6 +36,7 @@
 #include "gemm_direct.h"
 #include "gemm_f32.h"
 #include "gemm_pp_layout.h"
+#include "gemm_ring.h"
 #include "vx_lds_dma.hip.h"
 #include "vx_mfma16.hip.h"
 
@@ -894,7 +895,8 @@ struct SkSpace {
   char *base = nullptr;
   size_t bytes = 0;
   int seq = 0;
-  /* the register GEMM's split launches: tickets, then partial sums */
+  /* the split launches of the register GEMM and of 128x128 tiles: tickets,
+   * then partial sums */
   char *split = nullptr;
   size_t split_bytes = 0;
 };
@@ -999,6 +1001,24 @@ void launch_direct(const GemmArgs &g, hipStream_t s) {
   gemm_direct_launch(g, plan, sp.split, s);
 }
 
+void launch_ring(const GemmArgs &g, hipStream_t s) {
+  const int cus = device_cu_count();
+  int splits = ring::splits(g.m, g.n, g.k, cus, g.may_split);
+  if (splits == 1) {
+    gemm_ring_launch(g, 1, nullptr, s);
+    return;
+  }
+  std::lock_guard<std::mutex> hold(sk_mutex);
+  int dev = 0;
+  VX_HIP_CHECK(hipGetDevice(&dev));
+  SkSpace &sp = sk_spaces()[{dev, s}];
+  if (!sk_reserve(sp.split, sp.split_bytes, (size_t)ring::ws_bytes(g.m, g.n, splits),
+                  (size_t)ring::kTicketBytes, s)) {
+    splits = 1;
+  }
+  gemm_ring_launch(g, splits, sp.split, s);
+}
+
 /* Microseconds of the ping-pong launches on a 256-CU MI355X: 9 and, a round
  * of the CUs, 0.6 a stage of K while few CUs compute, up to 0.84 with all of
  * them (4096^3 113 us, 64 x 4096 x 4096 81). The stream-K tail counts as the
@@ -1046,6 +1066,8 @@ bool gemm_kernel_takes(GemmKernel which, const GemmArgs &g) {
     return tiled_takes(g);
   case GEMM_MFMA_DIRECT:
     return gemm_direct_takes(g);
+  case GEMM_MFMA_RING:
+    return pp_takes(g);
   default:
     return false;
   }
@@ -1054,19 +1076,33 @@ bool gemm_kernel_takes(GemmKernel which, const GemmArgs &g) {
 GemmKernel gemm_pick(const GemmArgs &g) {
   /* 16-bit products of 2^18 multiply-adds and K >= 128, or of 2^25: MFMA
    * kernels (smaller ones stay exact-order: a launch is most of their time,
-   * 64^3 6.0 us). 256x256 tiles or the register GEMM, whichever takes less
-   * time by its model: 512 x 4096 x 4096 88 and 33 us, 4096^3 113 and 215. */
+   * 64^3 6.0 us). Of the register GEMM and, where rows and K allow their
+   * loads, 128x128 and 256x256 tiles, the one of least time by its model:
+   * 512 x 4096 x 4096 34, 45 and 88 us, 1024 x 4096 x 4096 66, 49 and 90,
+   * 4096^3 215, 148 and 113. Grids of more than one round of 256x256 tiles
+   * keep them. */
   const double work = (double)g.m * (double)g.n * (double)g.k;
   if (work >= 33554432.0 || (g.k >= 128 && work >= 262144.0)) {
-    double us = 1e30;
+    GemmKernel which = GEMM_NONE;
+    double least = 1e30, us = 1e30;
     if (gemm_direct_takes(g)) {
-      (void)direct_plan(g, g.may_split, &us);
+      (void)direct_plan(g, g.may_split, &least);
+      which = GEMM_MFMA_DIRECT;
     }
-    if (pp_takes(g) && pp_us(g) <= us) {
-      return sk_takes(g) ? GEMM_MFMA_SK : GEMM_MFMA_PP;
+    if (pp_takes(g)) {
+      const int cus = device_cu_count();
+      const int64_t tiles = ((g.m + kTileM - 1) / kTileM) * ((g.n + kTileN - 1) / kTileN);
+      us = ring::us(g.m, g.n, g.k, ring::splits(g.m, g.n, g.k, cus, g.may_split), cus);
+      if (tiles <= cus && us < least) {
+        least = us;
+        which = GEMM_MFMA_RING;
+      }
+      if (pp_us(g) <= least) {
+        which = sk_takes(g) ? GEMM_MFMA_SK : GEMM_MFMA_PP;
+      }
     }
-    if (us < 1e30) {
-      return GEMM_MFMA_DIRECT;
+    if (which != GEMM_NONE) {
+      return which;
     }
   }
   /* f32: the exact-order kernel (bit-equal to the reference's host loop)
@@ -1100,6 +1136,11 @@ bool gemm_launch_kernel(GemmKernel which, const GemmArgs &g,
       return false;
     }
     launch_direct(g, stream);
+  } else if (which == GEMM_MFMA_RING) {
+    if (!pp_takes(g)) {
+      return false;
+    }
+    launch_ring(g, stream);
   } else if (which == GEMM_F32_MFMA) {
     if (!f32_mfma_takes(g)) {
       return false;

@@ -1,0 +1,62 @@
+/*
+ * gemm_ring.h -- launcher of the 128x128-tile GEMM (gemm_ring.hip) and the
+ * choice of its splits. Plain host arithmetic.
+ */
+#ifndef VX_AMD_GEMM_RING_H
+#define VX_AMD_GEMM_RING_H
+
+#include "../vx_kernels.h"
+
+#include <algorithm>
+
+namespace vxk {
+namespace ring {
+
+constexpr int kTile = 128;
+/* A split launch's workspace: a ticket per tile, zero between launches, then
+ * the partial sums. */
+constexpr int kMaxSplitTiles = 1024;
+constexpr int64_t kTicketBytes = kMaxSplitTiles * 4;
+
+inline int64_t tiles(int64_t m, int64_t n) {
+  return ((m + kTile - 1) / kTile) * ((n + kTile - 1) / kTile);
+}
+inline int64_t ws_bytes(int64_t m, int64_t n, int splits) {
+  return kTicketBytes + tiles(m, n) * splits * (int64_t)(kTile * kTile * 4);
+}
+
+/* Microseconds on a 256-CU MI355X: a stage of K takes 0.53 where CUs have two
+ * workgroups and 0.34 where they have one, a round of two per CU 2.5 to start
+ * and store, and a split its sums' way to memory and back. */
+inline double us(int64_t m, int64_t n, int64_t k, int splits, int cus) {
+  const int64_t units = tiles(m, n) * splits, slots = 2 * (int64_t)cus;
+  const int64_t full = units / slots, rest = units % slots;
+  const double stages = (double)(k / 32) / splits;
+  double t = 3.0 + 2.5 * (double)(full + (rest > 0));
+  t += stages * (0.53 * (double)full + (rest > cus ? 0.53 : rest > 0 ? 0.34 : 0.0));
+  if (splits > 1) {
+    t += 3.0 + (double)units * kTile * kTile * 8 / 5e6;
+  }
+  return t;
+}
+
+/* Splits of least time by that model. */
+inline int splits(int64_t m, int64_t n, int64_t k, int cus, bool may_split) {
+  int best = 1;
+  if (may_split && tiles(m, n) <= kMaxSplitTiles) {
+    for (int s = 2; s <= 8 && k / 32 / s >= 8; ++s) {
+      if (us(m, n, k, s, cus) < us(m, n, k, best, cus)) {
+        best = s;
+      }
+    }
+  }
+  return best;
+}
+
+} // namespace ring
+
+void gemm_ring_launch(const GemmArgs &g, int splits, char *ws, hipStream_t s);
+
+} // namespace vxk
+
+#endif /* VX_AMD_GEMM_RING_H */

@@ -46,11 +46,13 @@ enum GemmKernel {
                         (grids of 1 to 1.5 rounds; needs a workspace) */
   GEMM_MFMA_DIRECT = 11, /* bf16/f16 on 16x16x32 MFMAs fed from memory without
                             LDS: any alignment, few rows, small grids */
+  GEMM_MFMA_RING = 12, /* bf16/f16 on 16x16x32 MFMAs, 128x128 tiles, two to a
+                          CU: what GEMM_MFMA_PP takes, where its grid is small */
 };
 
 inline bool gemm_is_mfma(GemmKernel k) {
   return k == GEMM_MFMA_PP || k == GEMM_F32_MFMA || k == GEMM_MFMA_SK ||
-         k == GEMM_MFMA_DIRECT;
+         k == GEMM_MFMA_DIRECT || k == GEMM_MFMA_RING;
 }
 
 GemmKernel gemm_pick(const GemmArgs &g);
