@@ -58,6 +58,10 @@ struct LlamaI8 {
    * for) their logits. */
   float *px = nullptr, *pq = nullptr, *plogits = nullptr;
   uint16_t *pdim = nullptr, *phid = nullptr;
+  /* Two pieces of pinned memory that logits pass through on their way to the
+   * caller's (taken when logits are first asked for), and their arrivals. */
+  char *staging = nullptr;
+  hipEvent_t arrived[2] = {nullptr, nullptr};
   hipStream_t stream = nullptr;
   /* The instantiated step graphs (one step, kGraphSteps steps; [1]: for
    * steps whose positions are all below step_attention_near, whose
@@ -100,6 +104,14 @@ void release(LlamaI8 &m) {
   if (m.stream) {
     (void)hipStreamSynchronize(m.stream);
     (void)hipStreamDestroy(m.stream);
+  }
+  for (hipEvent_t e : m.arrived) {
+    if (e) {
+      (void)hipEventDestroy(e);
+    }
+  }
+  if (m.staging) {
+    (void)hipHostFree(m.staging);
   }
   for (void *p : m.owned) {
     (void)hipFree(p);
@@ -315,6 +327,36 @@ void enqueue_prefill(LlamaI8 &m, int pos0, int count) {
     w2.kp = hid_kp;
     w2.out = m.px;
     vxk::prefill_resid_launch(w2, m.stream);
+  }
+}
+
+/* `bytes` at `src` on the GPU to `dst` in the caller's memory, behind the
+ * model's stream. A piece is copied out of pinned memory while the next one
+ * arrives there: 25.6 MB in 0.75 ms, where a copy straight to pageable memory
+ * takes 1.5. */
+constexpr size_t kStagingPiece = 2 << 20;
+
+void read_back(LlamaI8 &m, char *dst, const char *src, size_t bytes) {
+  if (!m.staging) {
+    void *p = nullptr;
+    VX_HIP_CHECK(hipHostMalloc(&p, 2 * kStagingPiece));
+    m.staging = static_cast<char *>(p);
+    for (hipEvent_t &e : m.arrived) {
+      VX_HIP_CHECK(hipEventCreateWithFlags(&e, hipEventDisableTiming));
+    }
+  }
+  const size_t pieces = (bytes + kStagingPiece - 1) / kStagingPiece;
+  auto size = [&](size_t i) { return std::min(kStagingPiece, bytes - i * kStagingPiece); };
+  for (size_t i = 0; i <= pieces; ++i) {
+    if (i < pieces) {
+      VX_HIP_CHECK(hipMemcpyAsync(m.staging + i % 2 * kStagingPiece, src + i * kStagingPiece,
+                                  size(i), hipMemcpyDeviceToHost, m.stream));
+      VX_HIP_CHECK(hipEventRecord(m.arrived[i % 2], m.stream));
+    }
+    if (i > 0) {
+      VX_HIP_CHECK(hipEventSynchronize(m.arrived[(i - 1) % 2]));
+      memcpy(dst + (i - 1) * kStagingPiece, m.staging + (i - 1) % 2 * kStagingPiece, size(i - 1));
+    }
   }
 }
 
@@ -561,10 +603,9 @@ int32_t vx_llama_i8_logits(void *model, const int32_t *tokens, int32_t n,
       lg.out = m->plogits;
       vxk::prefill_logits_launch(lg, m->stream);
       VX_HIP_CHECK(hipGetLastError());
-      VX_HIP_CHECK(hipMemcpyAsync(logits + p * vocab, m->plogits, sizeof(float) * count * vocab,
-                                  hipMemcpyDeviceToHost, m->stream));
+      read_back(*m, reinterpret_cast<char *>(logits + p * vocab),
+                reinterpret_cast<const char *>(m->plogits), sizeof(float) * count * vocab);
     }
-    VX_HIP_CHECK(hipStreamSynchronize(m->stream));
     return VX_OP_OK;
   }
   vxk::step_start_launch(argmax_args(*m, n), m->stream);
