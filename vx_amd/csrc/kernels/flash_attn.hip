@@ -178,8 +178,10 @@ __device__ __forceinline__ uint32_t pack2(float lo, float hi) {
 }
 
 /* kQT query tiles of 32 per wave: a wave owns 32 * kQT queries, so each K
- * and V operand read from LDS feeds kQT MFMAs. */
-template <int kD, int kQT, int kBK, bool kSplit>
+ * and V operand read from LDS feeds kQT MFMAs. With kGroups = 2 the workgroup
+ * owns half as many queries; each half of its waves walks every other key
+ * block through a ring of its own, and the halves meet in LDS at the end. */
+template <int kD, int kQT, int kBK, bool kSplit, int kGroups>
 __global__ __launch_bounds__(kThreads, kQT == 1 ? 2 : 1) void flash_fwd(
     const uint16_t *__restrict__ Q, const uint16_t *__restrict__ K,
     const uint16_t *__restrict__ V, uint16_t *__restrict__ O,
@@ -191,20 +193,26 @@ __global__ __launch_bounds__(kThreads, kQT == 1 ? 2 : 1) void flash_fwd(
   constexpr int kKS = kBlockK / 16;               /* 16-key MFMA steps */
   constexpr int kChunks = kD / 8;                 /* 16-byte chunks per row */
   constexpr int kUnits = kBlockK * kChunks;       /* 16-byte units per plane */
-  constexpr int kLoads = kUnits / kThreads;       /* per thread per plane */
+  constexpr int kGroupThreads = kThreads / kGroups;
+  constexpr int kWavesQ = 4 / kGroups;            /* waves along the queries */
+  constexpr int kLoads = kUnits / kGroupThreads;  /* per thread per plane */
   constexpr int kDSteps = kD / 16;                /* MFMA k-steps over d */
   constexpr int kDTiles = kD / 32;                /* 32-wide d tiles of O^T */
   constexpr int kRowBytes = kD * 2;
   constexpr int kWaveQ = 32 * kQT;                /* queries per wave */
-  constexpr int kBlockQ = 4 * kWaveQ;             /* queries per workgroup */
-  /* [stage][K|V][unit] */
-  __shared__ u32x4 ring[2][2][kUnits];
+  constexpr int kBlockQ = kWavesQ * kWaveQ;       /* queries per workgroup */
+  static_assert(kGroups == 1 || (!kSplit && kQT == 1), "groups meet in LDS");
+  /* [group][stage][K|V][unit] */
+  __shared__ u32x4 ring[kGroups][2][2][kUnits];
 
   const int t = threadIdx.x;
   const int wave = __builtin_amdgcn_readfirstlane(t >> 6);
   const int lane = t & 63;
   const int lq = lane & 31;
   const int g = lane >> 5;
+  const int grp = kGroups == 1 ? 0 : __builtin_amdgcn_readfirstlane(wave / kWavesQ);
+  const int wq = kGroups == 1 ? wave : wave % kWavesQ;
+  const int tg = kGroups == 1 ? t : t % kGroupThreads;
 
   /* Launch order -> (head, query block). Workgroup i runs on XCD i % 8, so
    * each XCD gets every 8th head; it walks them kHeadGroup heads at a time
@@ -247,7 +255,7 @@ __global__ __launch_bounds__(kThreads, kQT == 1 ? 2 : 1) void flash_fwd(
   const int shift = seq_k - seq_q; /* query i sees keys <= i + shift */
 
   const int q0 = qb * kBlockQ;
-  const int qw0 = q0 + wave * kWaveQ;
+  const int qw0 = q0 + wq * kWaveQ;
 
   /* Keys any row of this workgroup may see, and this wave's last key. */
   int kv_end = seq_k;
@@ -258,6 +266,9 @@ __global__ __launch_bounds__(kThreads, kQT == 1 ? 2 : 1) void flash_fwd(
   }
   int nblocks = kv_end > 0 ? (kv_end + kBlockK - 1) / kBlockK : 0;
   int first = 0; /* first key block of this workgroup */
+  /* Groups take key blocks in turn: block `blk` of a group starts here. */
+  nblocks = (nblocks + kGroups - 1) / kGroups;
+  auto key_of = [&](int blk) { return (blk * kGroups + grp) * kBlockK; };
   if constexpr (kSplit) {
     const int per = ((seq_k + kBlockK - 1) / kBlockK + splits - 1) / splits;
     first = sp * per;
@@ -279,34 +290,37 @@ __global__ __launch_bounds__(kThreads, kQT == 1 ? 2 : 1) void flash_fwd(
     }
   }
 
-  /* Load offsets: unit u = (p * kThreads + t) of a plane is key u / kChunks,
+  /* Load offsets: unit u = (p * kGroupThreads + tg) of a plane is key u / kChunks,
    * physical chunk u % kChunks, filled from the logical chunk the swizzle
    * puts there. */
   uint32_t k_off[kLoads], v_off[kLoads];
 #pragma unroll
   for (int p = 0; p < kLoads; ++p) {
-    const int u = p * kThreads + t;
+    const int u = p * kGroupThreads + tg;
     const int key = u / kChunks;
     const int pc = u % kChunks;
     k_off[p] = (uint32_t)(key * kRowBytes + swz<kChunks>(key, pc) * 16);
     v_off[p] = (uint32_t)(key * kRowBytes + swz_v<kChunks>(key, pc) * 16);
   }
   const uint32_t ring_base =
-      (uint32_t)(uintptr_t)(VX_LDS void *)&ring[0][0][0];
+      (uint32_t)(uintptr_t)(VX_LDS void *)&ring[grp][0][0][0];
   /* Block b of K and of V lives in slot (b - first) % 2 of its plane
    * (counted from the workgroup's first block, so the loop below, which
    * steps two blocks at a time from there, sees constant slots). */
   auto issue = [&](int blk, int plane) {
-    const int key0 = blk * kBlockK;
-    const int bytes = min(kBlockK, seq_k - key0) * kRowBytes;
+    const int key0 = key_of(blk);
+    int bytes = min(kBlockK, seq_k - key0) * kRowBytes;
+    if constexpr (kGroups > 1) {
+      bytes = max(bytes, 0); /* the last group's turn may be past the end */
+    }
     const uint16_t *src = plane == 0 ? K : V;
     const i32x4 rs = buffer_rsrc(src + kv_base + (int64_t)key0 * kD, bytes);
     const uint32_t *off = plane == 0 ? k_off : v_off;
     const uint32_t base =
-        ring_base + (uint32_t)(((((blk - first) & 1) * 2 + plane) * kUnits + wave * 64) * 16);
+        ring_base + (uint32_t)(((((blk - first) & 1) * 2 + plane) * kUnits + wq * 64) * 16);
 #pragma unroll
     for (int p = 0; p < kLoads; ++p) {
-      dma16(rs, off[p], base + (uint32_t)(p * kThreads * 16));
+      dma16(rs, off[p], base + (uint32_t)(p * kGroupThreads * 16));
     }
   };
 
@@ -341,7 +355,7 @@ __global__ __launch_bounds__(kThreads, kQT == 1 ? 2 : 1) void flash_fwd(
   /* S^T of block `blk` for this wave: keys 32*kt + (row), queries of tile
    * qt; one K operand read feeds all query tiles. */
   auto scores = [&](int blk, Scores &st) {
-    const u32x4 *kl = ring[(blk - first) & 1][0];
+    const u32x4 *kl = ring[grp][(blk - first) & 1][0];
 #pragma unroll
     for (int ds = 0; ds < kDSteps; ++ds) {
 #pragma unroll
@@ -434,7 +448,7 @@ __global__ __launch_bounds__(kThreads, kQT == 1 ? 2 : 1) void flash_fwd(
         }
       }
     }
-    const VX_LDS char *vl = (const VX_LDS char *)&ring[(blk - first) & 1][1][0];
+    const VX_LDS char *vl = (const VX_LDS char *)&ring[grp][(blk - first) & 1][1][0];
 #pragma unroll
     for (int ks = 0; ks < kKS; ++ks) {
 #pragma unroll
@@ -488,13 +502,13 @@ __global__ __launch_bounds__(kThreads, kQT == 1 ? 2 : 1) void flash_fwd(
     if (blk + 1 < nblocks) {
       issue(blk + 1, 1);
     }
-    const int key0 = blk * kBlockK;
+    const int key0 = key_of(blk);
     if (key0 > wave_last) {
       return;
     }
     const bool need_mask =
         key0 + kBlockK > seq_k || (causal && key0 + kBlockK - 1 > qw0 + shift);
-    const bool next = blk + 1 < nblocks && key0 + kBlockK <= wave_last;
+    const bool next = blk + 1 < nblocks && key0 + kGroups * kBlockK <= wave_last;
     u32x4 pt[kQT][kKS];
     float alpha[kQT];
     bool bump[kQT];
@@ -569,7 +583,7 @@ __global__ __launch_bounds__(kThreads, kQT == 1 ? 2 : 1) void flash_fwd(
     }
     wait_all_loads();
     lds_barrier();
-    if (first * kBlockK <= wave_last) {
+    if (key_of(first) <= wave_last) {
       scores(first, sa);
     }
   }
@@ -577,6 +591,46 @@ __global__ __launch_bounds__(kThreads, kQT == 1 ? 2 : 1) void flash_fwd(
     step(blk, sa, sb);
     if (blk + 1 < nblocks) {
       step(blk + 1, sb, sa);
+    }
+  }
+
+  if constexpr (kGroups == 2) {
+    /* Group 1 leaves its max, sum and output in LDS, lane by lane; group 0's
+     * wave of the same queries takes them in. */
+    f32x4v *so = reinterpret_cast<f32x4v *>(&ring[0][0][0][0]) + wq * (kDTiles * 4 + 1) * 64 + lane;
+    __syncthreads();
+    if (grp == 1) {
+#pragma unroll
+      for (int i = 0; i < kDTiles; ++i) {
+#pragma unroll
+        for (int r4 = 0; r4 < 4; ++r4) {
+          so[(4 * i + r4) * 64] = f32x4v{o_acc[0][i][4 * r4], o_acc[0][i][4 * r4 + 1],
+                                         o_acc[0][i][4 * r4 + 2], o_acc[0][i][4 * r4 + 3]};
+        }
+      }
+      so[kDTiles * 4 * 64] = f32x4v{m_run[0], l_run[0], 0.0f, 0.0f};
+    }
+    __syncthreads();
+    if (grp == 1) {
+      return;
+    }
+    const f32x4v other = so[kDTiles * 4 * 64];
+    const float mx = fmaxf(m_run[0], other[0]);
+    const float m_use = mx == -INFINITY ? 0.0f : mx;
+    const float f0 = __builtin_amdgcn_exp2f(m_run[0] - m_use);
+    const float f1 = __builtin_amdgcn_exp2f(other[0] - m_use);
+    m_run[0] = mx;
+    l_run[0] = l_run[0] * f0 + other[1] * f1;
+#pragma unroll
+    for (int i = 0; i < kDTiles; ++i) {
+#pragma unroll
+      for (int r4 = 0; r4 < 4; ++r4) {
+        const f32x4v v = so[(4 * i + r4) * 64];
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          o_acc[0][i][4 * r4 + e] = o_acc[0][i][4 * r4 + e] * f0 + v[e] * f1;
+        }
+      }
     }
   }
 
@@ -698,17 +752,24 @@ template <int kD, int kQT, int kBK>
 void launch(const uint16_t *q, const uint16_t *k, const uint16_t *v,
             uint16_t *o, float *lse, int heads, int group, int seq_q, int seq_k,
             int bh, float scale_log2, bool causal, int splits, float *opart,
-            float *lpart, hipStream_t stream) {
+            float *lpart, hipStream_t stream) { /* splits 0: two groups */
+  if (splits == 0) {
+    const int qblocks64 = (seq_q + 63) / 64;
+    hipLaunchKernelGGL((flash_fwd<kD, 1, kBK, false, 2>), dim3((unsigned)(bh * qblocks64)),
+                       dim3(kThreads), 0, stream, q, k, v, o, lse, heads, group, seq_q, seq_k, bh,
+                       qblocks64, scale_log2, causal, 1, nullptr, nullptr);
+    return;
+  }
   constexpr int kBlockQ = 4 * 32 * kQT;
   const int qblocks = (seq_q + kBlockQ - 1) / kBlockQ;
   if (splits <= 1) {
-    hipLaunchKernelGGL((flash_fwd<kD, kQT, kBK, false>),
+    hipLaunchKernelGGL((flash_fwd<kD, kQT, kBK, false, 1>),
                        dim3((unsigned)(bh * qblocks)), dim3(kThreads), 0, stream,
                        q, k, v, o, lse, heads, group, seq_q, seq_k, bh, qblocks,
                        scale_log2, causal, 1, nullptr, nullptr);
     return;
   }
-  hipLaunchKernelGGL((flash_fwd<kD, kQT, kBK, true>),
+  hipLaunchKernelGGL((flash_fwd<kD, kQT, kBK, true, 1>),
                      dim3((unsigned)(bh * qblocks * splits)), dim3(kThreads), 0,
                      stream, q, k, v, o, lse, heads, group, seq_q, seq_k, bh,
                      qblocks, scale_log2, causal, splits, opart, lpart);
@@ -726,17 +787,41 @@ std::atomic<int> forced_splits{0};
  * (measured on the 512-query prefill chunks, 128 items: over 2048 keys 2
  * splits 35.5 us against 37.6 for 4; over 8192 keys 4 splits 88.8 us against
  * 100.7 for 2 and 98-101 for 6 and 8; over 512 keys no split pays). */
-int pick_splits(int64_t items, int64_t key_blocks, int cus) {
-  const int forced = forced_splits.load();
-  if (forced > 0) {
-    return (int)std::min<int64_t>(forced, std::max<int64_t>(key_blocks, 1));
-  }
+int auto_splits(int64_t items, int64_t key_blocks, int cus) {
   const int64_t slots = 2 * (int64_t)cus;
   if (items >= slots) {
     return 1;
   }
   const int64_t want = (slots + items - 1) / items;
   return (int)std::max<int64_t>(1, std::min<int64_t>({want, 8, key_blocks / 16}));
+}
+
+int pick_splits(int64_t items, int64_t key_blocks, int cus) {
+  const int forced = forced_splits.load();
+  if (forced > 0) {
+    return (int)std::min<int64_t>(forced, std::max<int64_t>(key_blocks, 1));
+  }
+  return auto_splits(items, key_blocks, cus);
+}
+
+/* Whether workgroups of 64 queries, whose two halves divide the keys, take the
+ * call: `items` 128-query and `items64` 64-query workgroups. They give a small
+ * grid twice the workgroups without partial results in memory, and load each
+ * key twice as often. Head size 64 (two to a CU): up to one round, where the
+ * keys would be cut less than four ways (16 heads, 2048^2 causal 33.3 -> 21.8
+ * us, 8 heads, 1000^2 18.0 -> 12.0; 1024 workgroups, 2 x 32 heads, 1024^2 30.1
+ * against 33.5; 128 queries of 32 heads over 8000 keys in 8 splits 28.1
+ * against 61). Head size 128 (one to a CU): up to one round, where the keys
+ * would not be cut (8 heads, 1000^2 24.2 -> 19.0; 512 queries of 32 heads over
+ * 512 keys 15.9 -> 13.5, over 2048 in 2 splits 36.0 against 35.1, over 8192 in
+ * 4 splits 87 against 125). */
+bool two_groups(int head_dim, int64_t items, int64_t items64, int64_t key_blocks, int cus,
+                bool allow_split) {
+  if (allow_split && forced_splits.load() > 1) {
+    return false;
+  }
+  const int splits = auto_splits(items, key_blocks, cus);
+  return head_dim == 64 ? items64 <= 2 * cus && splits < 4 : items64 <= cus && splits == 1;
 }
 
 /* Split partials of one (device, stream). Launches on one stream run in
@@ -916,6 +1001,10 @@ bool flash_attn_fwd_launch(const uint16_t *q, const uint16_t *k,
   if (items * splits > INT32_MAX || bh * seq_q * (head_dim / 4) > INT32_MAX) {
     splits = 1;
   }
+  if (two_groups((int)head_dim, items, bh * ((seq_q + 63) / 64), key_blocks, device_cu_count(),
+                 allow_split)) {
+    splits = 0;
+  }
   if (splits > 1) {
     /* Held from the workspace lookup through the launch, so a growth on one
      * thread cannot free a block another thread's launch is about to use. */
@@ -947,11 +1036,11 @@ bool flash_attn_fwd_launch(const uint16_t *q, const uint16_t *k,
   }
   if (head_dim == 128) {
     launch<128, VX_FA_QT, VX_FA_BK>(q, k, v, o, lse, (int)heads, group, (int)seq_q,
-                          (int)seq_k, (int)bh, scale_log2, causal, 1, nullptr,
+                          (int)seq_k, (int)bh, scale_log2, causal, splits, nullptr,
                           nullptr, stream);
   } else {
     launch<64, VX_FA_QT, VX_FA_BK>(q, k, v, o, lse, (int)heads, group, (int)seq_q,
-                         (int)seq_k, (int)bh, scale_log2, causal, 1, nullptr,
+                         (int)seq_k, (int)bh, scale_log2, causal, splits, nullptr,
                          nullptr, stream);
   }
   VX_HIP_CHECK(hipGetLastError());
