@@ -48,7 +48,8 @@ def check(c, a, b):
 
 
 @pytest.mark.parametrize("m,n,k", [(1, 1, 1), (128, 128, 31), (129, 127, 32), (127, 130, 33), (5, 300, 64),
-                                   (300, 5, 95), (256, 384, 96), (130, 131, 129), (200, 200, 1000)])
+                                   (300, 5, 95), (256, 384, 96), (130, 131, 129), (200, 200, 1000),
+                                   (130, 131, 2047), (20, 1000, 4100)])
 @pytest.mark.parametrize("pad", [0, 1])
 def test_edges_of_stages_and_tiles(hiplib, rng, m, n, k, pad):
     announce(f"f32 gemm {m}x{n}x{k} pad {pad}")
@@ -89,6 +90,22 @@ def test_rows_and_columns_too_small_for_the_planes(hiplib, rng):
     c = product(hiplib, a, b)
     check(c, a, b)
     assert not c[141].any()
+
+
+def test_tiny_and_infinite_rows_over_splits(hiplib, rng):
+    """K divided over workgroups: a row that is tiny in some of its splits
+    only, one that is tiny in all, one with an infinity in one split."""
+    announce("f32 gemm, splits, tiny and infinite rows")
+    m, n, k = 200, 140, 3000
+    a = rng.uniform(-1, 1, (m, k)).astype(np.float32)
+    b = rng.uniform(-1, 1, (k, n)).astype(np.float32)
+    a[20, :2000] *= np.float32(2.0 ** -118)
+    a[30] *= np.float32(2.0 ** -118)
+    check(product(hiplib, a, b), a, b)
+    a[199, 2500] = np.inf
+    c = product(hiplib, a, b)
+    check(c[:199], a[:199], b)
+    assert np.array_equal(c[199], np.where(b[2500] > 0, np.inf, -np.inf))
 
 
 def test_infinities_and_nans(hiplib, rng):

@@ -895,8 +895,8 @@ struct SkSpace {
   char *base = nullptr;
   size_t bytes = 0;
   int seq = 0;
-  /* the split launches of the register GEMM and of 128x128 tiles: tickets,
-   * then partial sums */
+  /* the split launches of the register GEMM, of 128x128 tiles and of f32:
+   * tickets, then partial sums */
   char *split = nullptr;
   size_t split_bytes = 0;
 };
@@ -983,40 +983,46 @@ direct::Plan direct_plan(const GemmArgs &g, bool may_split, double *us) {
   return direct::plan(g.m, g.n, g.k, odd, device_cu_count(), may_split, us);
 }
 
-void launch_direct(const GemmArgs &g, hipStream_t s) {
-  double us;
-  direct::Plan plan = direct_plan(g, g.may_split, &us);
-  if (!plan.ws_bytes) {
-    gemm_direct_launch(g, plan, nullptr, s);
-    return;
-  }
-  std::lock_guard<std::mutex> hold(sk_mutex);
+/* The split workspace of `s`, of `bytes`, for the launches that keep tickets in
+ * its first kTicketBytes; null when there is none to be had. The caller holds
+ * sk_mutex, through its launch. */
+static_assert(ring::kTicketBytes == direct::kTicketBytes &&
+                  f32::kTicketBytes == direct::kTicketBytes,
+              "one workspace for all of them");
+char *split_space(size_t bytes, hipStream_t s) {
   int dev = 0;
   VX_HIP_CHECK(hipGetDevice(&dev));
   SkSpace &sp = sk_spaces()[{dev, s}];
-  if (!sk_reserve(sp.split, sp.split_bytes, (size_t)plan.ws_bytes, (size_t)direct::kTicketBytes,
-                  s)) {
-    plan = direct_plan(g, false, &us);
-  }
-  gemm_direct_launch(g, plan, sp.split, s);
+  return sk_reserve(sp.split, sp.split_bytes, bytes, (size_t)direct::kTicketBytes, s) ? sp.split
+                                                                                       : nullptr;
 }
 
 void launch_ring(const GemmArgs &g, hipStream_t s) {
-  const int cus = device_cu_count();
-  int splits = ring::splits(g.m, g.n, g.k, cus, g.may_split);
-  if (splits == 1) {
-    gemm_ring_launch(g, 1, nullptr, s);
-    return;
-  }
+  const int splits = ring::splits(g.m, g.n, g.k, device_cu_count(), g.may_split);
   std::lock_guard<std::mutex> hold(sk_mutex);
-  int dev = 0;
-  VX_HIP_CHECK(hipGetDevice(&dev));
-  SkSpace &sp = sk_spaces()[{dev, s}];
-  if (!sk_reserve(sp.split, sp.split_bytes, (size_t)ring::ws_bytes(g.m, g.n, splits),
-                  (size_t)ring::kTicketBytes, s)) {
-    splits = 1;
+  char *ws = splits > 1 ? split_space((size_t)ring::ws_bytes(g.m, g.n, splits), s) : nullptr;
+  gemm_ring_launch(g, ws ? splits : 1, ws, s);
+}
+
+void launch_f32(const GemmArgs &g, hipStream_t s) {
+  const int splits = f32::splits(g.m, g.n, g.k, device_cu_count(), g.may_split);
+  std::lock_guard<std::mutex> hold(sk_mutex);
+  char *ws = splits > 1 ? split_space((size_t)(f32::kTicketBytes + f32::tiles(g.m, g.n) * splits *
+                                                                       (int64_t)f32::kPart),
+                                      s)
+                        : nullptr;
+  gemm_f32_launch(g, ws ? splits : 1, ws, s);
+}
+
+void launch_direct(const GemmArgs &g, hipStream_t s) {
+  double us;
+  direct::Plan plan = direct_plan(g, g.may_split, &us);
+  std::lock_guard<std::mutex> hold(sk_mutex);
+  char *ws = plan.ws_bytes ? split_space((size_t)plan.ws_bytes, s) : nullptr;
+  if (plan.ws_bytes && !ws) {
+    plan = direct_plan(g, false, &us);
   }
-  gemm_ring_launch(g, splits, sp.split, s);
+  gemm_direct_launch(g, plan, ws, s);
 }
 
 /* Microseconds of the ping-pong launches on a 256-CU MI355X: 9 and, a round
@@ -1106,8 +1112,10 @@ GemmKernel gemm_pick(const GemmArgs &g) {
     }
   }
   /* f32: the exact-order kernel (bit-equal to the reference's host loop)
-   * below 2^30 multiply-adds, the MFMA kernel above. */
-  if (g.m >= 128 && g.n >= 128 && (double)g.m * g.n * g.k >= 1073741824.0 &&
+   * below 2^30 multiply-adds, the MFMA kernel above, also where most of its
+   * tile is past the last row (10 x 12000 x 12000 553 -> 239 us, 100 x 4000 x
+   * 4000 188 -> 36). */
+  if (g.m >= 8 && g.n >= 8 && (double)g.m * g.n * g.k >= 1073741824.0 &&
       f32_mfma_takes(g)) {
     return GEMM_F32_MFMA;
   }
@@ -1145,7 +1153,7 @@ bool gemm_launch_kernel(GemmKernel which, const GemmArgs &g,
     if (!f32_mfma_takes(g)) {
       return false;
     }
-    gemm_f32_launch(g, stream);
+    launch_f32(g, stream);
   } else if (which == GEMM_TILED) {
     if (!tiled_takes(g)) {
       return false;

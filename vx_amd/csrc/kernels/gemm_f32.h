@@ -1,5 +1,6 @@
 /*
- * gemm_f32.h -- launcher of the f32 MFMA GEMM (gemm_f32.hip).
+ * gemm_f32.h -- launcher of the f32 MFMA GEMM (gemm_f32.hip) and the choice of
+ * its splits. Plain host arithmetic.
  */
 #ifndef VX_AMD_GEMM_F32_H
 #define VX_AMD_GEMM_F32_H
@@ -8,9 +9,45 @@
 
 namespace vxk {
 namespace f32 {
+
 constexpr int kTile = 128;
+/* A split launch's workspace: a ticket per tile, zero between launches, then
+ * each split's sums and magnitudes. */
+constexpr int kMaxSplitTiles = 1024;
+constexpr int64_t kTicketBytes = kMaxSplitTiles * 4;
+constexpr int kPart = (kTile * kTile + 2 * kTile) * 4;
+
+inline int64_t tiles(int64_t m, int64_t n) {
+  return ((m + kTile - 1) / kTile) * ((n + kTile - 1) / kTile);
 }
-void gemm_f32_launch(const GemmArgs &g, hipStream_t s);
+
+/* Splits of least time on a 256-CU MI355X (one workgroup to a CU): 1.15 us a
+ * stage of K, 4 a round, and for a split its sums' way to memory and back. */
+inline int splits(int64_t m, int64_t n, int64_t k, int cus, bool may_split) {
+  const int64_t t = tiles(m, n), stages = (k + 31) / 32;
+  if (!may_split || t > kMaxSplitTiles) {
+    return 1;
+  }
+  int best = 1;
+  double least = 1e30;
+  for (int s = 1; s <= 16 && (s == 1 || stages / s >= 4); ++s) {
+    const double rounds = (double)((t * s + cus - 1) / cus);
+    double us = rounds * (4.0 + 1.15 * (double)stages / s);
+    if (s > 1) {
+      us += 3.0 + (double)(t * s) * kPart * 2 / 5e6;
+    }
+    if (us < least) {
+      least = us;
+      best = s;
+    }
+  }
+  return best;
+}
+
+} // namespace f32
+
+void gemm_f32_launch(const GemmArgs &g, int splits, char *ws, hipStream_t s);
+
 } // namespace vxk
 
 #endif /* VX_AMD_GEMM_F32_H */

@@ -25,9 +25,10 @@
  * multiplies, costs a barrier more and gave the same: 108 us).
  *
  * Against f32 MFMAs in the same tile: 2048^3 248 -> 92 us with new inputs each
- * pass (188 TFLOP/s), 258 -> 106 with the same ones, 1024^3 125 -> 45, 128 x
- * 4096 x 4096 454 -> 142; error against 64 bits 8.1e-7 -> 2.5e-7 at 2048^3,
- * 1.1e-6 -> 3.8e-7 at K = 4096.
+ * pass (188 TFLOP/s), 258 -> 104 with the same ones; error against 64 bits
+ * 8.1e-7 -> 2.5e-7 at 2048^3, 1.1e-6 -> 3.8e-7 at K = 4096. Grids of fewer
+ * tiles than CUs divide K over workgroups: 1024^3 125 -> 27 us (undivided 45),
+ * 128 x 4096 x 4096 454 -> 38 (142).
  */
 #include "../vx_hip_common.h"
 #include "../vx_kernels.h"
@@ -77,7 +78,8 @@ __device__ __forceinline__ void split8(const float (&x)[8], u32x4 (&p)[3]) {
 
 __global__ __launch_bounds__(kThreads, 2) void gemm_f32_mfma(
     const float *__restrict__ A, const float *__restrict__ B, float *__restrict__ C, int64_t M,
-    int64_t N, int64_t K, int64_t lda, int64_t ldb, int64_t ldc, int tiles_m, int tiles_n) {
+    int64_t N, int64_t K, int64_t lda, int64_t ldb, int64_t ldc, int tiles_m, int tiles_n,
+    int splits, char *__restrict__ ws) {
   __shared__ u32x4 lds[2][2][3][kPlane]; /* [slot][A, B][plane] */
   const int t = threadIdx.x;
   const int lane = t & 63;
@@ -85,7 +87,10 @@ __global__ __launch_bounds__(kThreads, 2) void gemm_f32_mfma(
   const int l16 = lane & 15;
   const int g = lane >> 4;
   const int wm = wave >> 2, wn = wave & 3;
-  const pp::Tile tile = pp::tile_of(blockIdx.x, gridDim.x, tiles_m, tiles_n);
+  const int tiles = tiles_m * tiles_n;
+  const int split = (int)blockIdx.x / tiles;
+  const int id = (int)blockIdx.x - split * tiles;
+  const pp::Tile tile = pp::tile_of(id, tiles, tiles_m, tiles_n);
   const int64_t m0 = (int64_t)tile.tm * kTile;
   const int64_t n0 = (int64_t)tile.tn * kTile;
 
@@ -94,9 +99,15 @@ __global__ __launch_bounds__(kThreads, 2) void gemm_f32_mfma(
   const int a_row = t >> 2, a_chunk = t & 3;
   const int b_col = t & 127;
   const int b_chunk = wave >> 1;
-  const float *pa = A + min(m0 + a_row, M - 1) * lda + 8 * a_chunk;
+  /* this workgroup's stages */
+  const int64_t all = (K + kKs - 1) / kKs;
+  const int64_t first = all * split / splits;
+  const int64_t stages = all * (split + 1) / splits - first;
+  const int64_t whole = min(first + stages, K / kKs) - first;
+  const int64_t left = K - first * kKs; /* k from its first on */
+  const float *pa = A + min(m0 + a_row, M - 1) * lda + first * kKs + 8 * a_chunk;
   const int b_off = (int)(min(n0 + b_col, N - 1) - n0);
-  const float *pb = B + 8 * b_chunk * ldb + n0;
+  const float *pb = B + (first * kKs + 8 * b_chunk) * ldb + n0;
 
   auto load = [&](Regs &r, int64_t st) {
     const float *a = pa + st * kKs;
@@ -119,8 +130,8 @@ __global__ __launch_bounds__(kThreads, 2) void gemm_f32_mfma(
     const float *b = pb + st * kKs * ldb;
 #pragma unroll
     for (int e = 0; e < 8; ++e) {
-      r.a[e] = st * kKs + 8 * a_chunk + e < K ? a[e] : 0.0f;
-      r.b[e] = st * kKs + 8 * b_chunk + e < K ? (b + e * ldb)[b_off] : 0.0f;
+      r.a[e] = st * kKs + 8 * a_chunk + e < left ? a[e] : 0.0f;
+      r.b[e] = st * kKs + 8 * b_chunk + e < left ? (b + e * ldb)[b_off] : 0.0f;
     }
   };
   float a_max = 0.0f, b_max = 0.0f; /* of the row's and column's magnitudes */
@@ -185,7 +196,6 @@ __global__ __launch_bounds__(kThreads, 2) void gemm_f32_mfma(
     add(2, 0, lo);
   };
 
-  const int64_t stages = (K + kKs - 1) / kKs, whole = K / kKs;
   auto load_any = [&](Regs &r, int64_t st) {
     if (st < whole) {
       load(r, st);
@@ -252,6 +262,82 @@ __global__ __launch_bounds__(kThreads, 2) void gemm_f32_mfma(
   for (int c = 0; c < 4; ++c) {
     b_max = fmaxf(b_max, cols[c * kTile + b_col]);
   }
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+#pragma unroll
+    for (int j = 0; j < 2; ++j) {
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        hi[i][j][e] = hi[i][j][e] + lo[i][j][e];
+      }
+    }
+  }
+  if (splits > 1) {
+    /* The sums, then the magnitudes, go past the caches that other XCDs do not
+     * see; the workgroup with the last ticket adds all of them up in order. */
+    const __amdgpu_buffer_rsrc_t wr = __builtin_amdgcn_make_buffer_rsrc(
+        (void *)(ws + f32::kTicketBytes + (int64_t)id * splits * f32::kPart), (short)0,
+        splits * f32::kPart, 0x00020000);
+    constexpr int kMax = kTile * kTile * 4; /* [128] of the rows, [128] of the columns */
+    const int at = t * 16;
+    __shared__ int last;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+#pragma unroll
+      for (int j = 0; j < 2; ++j) {
+        __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, hi[i][j]), wr,
+                                               at + (2 * i + j) * kThreads * 16,
+                                               split * f32::kPart, 16 /* sc1 */);
+      }
+    }
+    if (a_chunk == 0) {
+      __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(a_max), wr, kMax + a_row * 4,
+                                            split * f32::kPart, 16 /* sc1 */);
+    }
+    if (b_chunk == 0) {
+      __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(b_max), wr,
+                                            kMax + (kTile + b_col) * 4, split * f32::kPart,
+                                            16 /* sc1 */);
+    }
+    __builtin_amdgcn_s_waitcnt(0);
+    __syncthreads();
+    int *ticket = reinterpret_cast<int *>(ws) + id;
+    if (t == 0) {
+      const int n = __hip_atomic_fetch_add(ticket, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      last = n == splits - 1;
+      if (n == splits - 1) { /* for the next launch */
+        __hip_atomic_store(ticket, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      }
+    }
+    __syncthreads();
+    if (!last) {
+      return;
+    }
+    a_max = b_max = 0.0f;
+    for (int s = 0; s < splits; ++s) {
+      f32x4 v[4][2];
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+#pragma unroll
+        for (int j = 0; j < 2; ++j) {
+          v[i][j] = __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(
+                                                  wr, at + (2 * i + j) * kThreads * 16,
+                                                  s * f32::kPart, 16 /* sc1 */));
+        }
+      }
+      a_max = fmaxf(a_max, __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(
+                               wr, kMax + a_row * 4, s * f32::kPart, 16 /* sc1 */)));
+      b_max = fmaxf(b_max, __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(
+                               wr, kMax + (kTile + b_col) * 4, s * f32::kPart, 16 /* sc1 */)));
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+#pragma unroll
+        for (int j = 0; j < 2; ++j) {
+          hi[i][j] = s == 0 ? v[i][j] : hi[i][j] + v[i][j];
+        }
+      }
+    }
+  }
   if (!__syncthreads_or(odd(a_max) || odd(b_max))) {
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
@@ -261,18 +347,13 @@ __global__ __launch_bounds__(kThreads, 2) void gemm_f32_mfma(
         const int64_t col = n0 + 32 * wn + 16 * j + 4 * g;
         if (row < M && col < N) {
           float *c = C + row * ldc + col;
-          f32x4 v;
-#pragma unroll
-          for (int e = 0; e < 4; ++e) {
-            v[e] = hi[i][j][e] + lo[i][j][e];
-          }
           if (col + 3 < N) {
-            reinterpret_cast<Four *>(c)->v = v;
+            reinterpret_cast<Four *>(c)->v = hi[i][j];
           } else {
 #pragma unroll
             for (int e = 0; e < 3; ++e) {
               if (col + e < N) {
-                c[e] = v[e];
+                c[e] = hi[i][j][e];
               }
             }
           }
@@ -337,12 +418,12 @@ __global__ __launch_bounds__(kThreads, 2) void gemm_f32_mfma(
 
 } // namespace
 
-void gemm_f32_launch(const GemmArgs &g, hipStream_t s) {
+void gemm_f32_launch(const GemmArgs &g, int splits, char *ws, hipStream_t s) {
   const int tiles_m = (int)((g.m + kTile - 1) / kTile), tiles_n = (int)((g.n + kTile - 1) / kTile);
-  hipLaunchKernelGGL(gemm_f32_mfma, dim3((unsigned)(tiles_m * tiles_n)), dim3(kThreads), 0, s,
+  hipLaunchKernelGGL(gemm_f32_mfma, dim3((unsigned)(tiles_m * tiles_n * splits)), dim3(kThreads), 0, s,
                      static_cast<const float *>(g.a), static_cast<const float *>(g.b),
                      static_cast<float *>(g.c), g.m, g.n, g.k, g.lda, g.ldb, g.ldc, tiles_m,
-                     tiles_n);
+                     tiles_n, splits, ws);
 }
 
 } // namespace vxk
