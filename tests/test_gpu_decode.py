@@ -241,6 +241,10 @@ def position_logits(cfg, weights, tokens):
     # heads of 2, K of 16 and 48; the fewest positions that go together, a
     # second tile of 16 with one position, and the whole cache
     (LlamaConfig(dim=16, hidden_dim=48, n_layers=2, n_heads=8, n_kv_heads=4, vocab_size=34,
+                 seq_len=40), 2),
+    (LlamaConfig(dim=16, hidden_dim=48, n_layers=2, n_heads=8, n_kv_heads=4, vocab_size=34,
+                 seq_len=40), 3),
+    (LlamaConfig(dim=16, hidden_dim=48, n_layers=2, n_heads=8, n_kv_heads=4, vocab_size=34,
                  seq_len=40), 4),
     (LlamaConfig(dim=16, hidden_dim=48, n_layers=2, n_heads=8, n_kv_heads=4, vocab_size=34,
                  seq_len=40), 17),

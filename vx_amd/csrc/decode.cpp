@@ -33,9 +33,11 @@ namespace {
 #endif
 constexpr int kGraphSteps = VX_DEC_GRAPH_STEPS;
 /* Given positions from which they go together (prefill) rather than step by
- * step: at the dim-768, 12-layer decoder a step takes 185 us, up to 16
- * positions together with one classified 547 us. */
-constexpr int kPrefillMin = 4;
+ * step, in a prompt and in a scored text: at the dim-768, 12-layer decoder 2,
+ * 3 and 4 prompt tokens and one new one take 418, 624 and 803 us in steps and
+ * 525 together; the logits of 1, 2 and 3 tokens 295, 541 and 802, and 525. */
+constexpr int kPrefillMin = 3;
+constexpr int kScoreMin = 2;
 
 struct LlamaI8 {
   vx_llama_i8_config cfg;
@@ -339,7 +341,12 @@ constexpr size_t kStagingPiece = 2 << 20;
 void read_back(LlamaI8 &m, char *dst, const char *src, size_t bytes) {
   if (!m.staging) {
     void *p = nullptr;
-    VX_HIP_CHECK(hipHostMalloc(&p, 2 * kStagingPiece));
+    if (hipHostMalloc(&p, 2 * kStagingPiece) != hipSuccess) {
+      (void)hipGetLastError();
+      VX_HIP_CHECK(hipMemcpyAsync(dst, src, bytes, hipMemcpyDeviceToHost, m.stream));
+      VX_HIP_CHECK(hipStreamSynchronize(m.stream));
+      return;
+    }
     m.staging = static_cast<char *>(p);
     for (hipEvent_t &e : m.arrived) {
       VX_HIP_CHECK(hipEventCreateWithFlags(&e, hipEventDisableTiming));
@@ -464,7 +471,7 @@ void *vx_llama_i8_create(const vx_llama_i8_config *cfg,
   m->hb = alloc<float>(*m, H);
   m->pos = alloc<int>(*m, 1);
   m->best = alloc<vxk::StepBest>(*m, (size_t)vxk::step_logits_groups(c.vocab_size));
-  if (c.seq_len >= kPrefillMin) {
+  if (c.seq_len >= kScoreMin) {
     /* one block: x and q, then the planes, whose columns past the width stay 0 */
     const size_t cap = vxk::kPrefillCap;
     const size_t pdim = (size_t)vxk::prefill_planes(c.dim);
@@ -583,7 +590,7 @@ int32_t vx_llama_i8_logits(void *model, const int32_t *tokens, int32_t n,
   VX_HIP_CHECK(hipMemcpyAsync(m->prompt, tokens, sizeof(int) * n,
                               hipMemcpyHostToDevice, m->stream));
   const size_t vocab = (size_t)m->cfg.vocab_size;
-  if (n >= kPrefillMin) {
+  if (n >= kScoreMin) {
     if (!m->plogits) {
       m->plogits =
           alloc<float>(*m, (size_t)std::min(vxk::kPrefillCap, m->cfg.seq_len) * vocab);
