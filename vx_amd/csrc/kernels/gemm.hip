@@ -1080,22 +1080,24 @@ bool gemm_kernel_takes(GemmKernel which, const GemmArgs &g) {
 }
 
 GemmKernel gemm_pick(const GemmArgs &g) {
-  /* 16-bit products of 2^18 multiply-adds and K >= 128, or of 2^25: MFMA
-   * kernels (smaller ones stay exact-order: a launch is most of their time,
+  /* 16-bit products of 2^18 multiply-adds and K >= 128, of 2^25, or of 2^24
+   * where rows and K allow the tiles' loads: MFMA kernels (smaller ones stay exact-order: a launch is most of their time,
    * 64^3 6.0 us). Of the register GEMM and, where rows and K allow their
    * loads, 128x128 and 256x256 tiles, the one of least time by its model:
    * 512 x 4096 x 4096 34, 45 and 88 us, 1024 x 4096 x 4096 66, 49 and 90,
    * 4096^3 215, 148 and 113. Grids of more than one round of 256x256 tiles
    * keep them. */
   const double work = (double)g.m * (double)g.n * (double)g.k;
-  if (work >= 33554432.0 || (g.k >= 128 && work >= 262144.0)) {
+  const bool tiles_ok = pp_takes(g);
+  if (work >= 33554432.0 || (g.k >= 128 && work >= 262144.0) ||
+      (tiles_ok && g.m >= 64 && g.n >= 64 && work >= 16777216.0)) {
     GemmKernel which = GEMM_NONE;
     double least = 1e30, us = 1e30;
     if (gemm_direct_takes(g)) {
       (void)direct_plan(g, g.may_split, &least);
       which = GEMM_MFMA_DIRECT;
     }
-    if (pp_takes(g)) {
+    if (tiles_ok) {
       const int cus = device_cu_count();
       const int64_t tiles = ((g.m + kTileM - 1) / kTileM) * ((g.n + kTileN - 1) / kTileN);
       us = ring::us(g.m, g.n, g.k, ring::splits(g.m, g.n, g.k, cus, g.may_split), cus);
