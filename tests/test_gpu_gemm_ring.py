@@ -1,4 +1,4 @@
-"""The 128x128-tile GEMM (gemm_ring.hip) at the edges of its tiles, ring and
+"""The 128x128- and 256x128-tile GEMM (gemm_ring.hip) at the edges of its tiles, ring and
 splits, against the f64 product, with the bound of f32 sums in any order."""
 
 import numpy as np
@@ -16,7 +16,8 @@ pytestmark = pytest.mark.gpu
     (1, 8, 32), (128, 128, 64), (127, 136, 96), (129, 264, 160),  # 1, 2, 3 and 5 stages of the ring
     (257, 120, 192), (640, 1000, 1024),  # 6 stages, 32 and a tile per two CUs
     (300, 264, 8192), (512, 1024, 4096),  # split along k
-    (1200, 4104, 288)])  # more tiles than CUs
+    (1200, 4104, 288),  # more tiles than CUs
+    (300, 11000, 2048), (2049, 2040, 2080)])  # 256x128 tiles, 64 and 65 stages
 @pytest.mark.parametrize("dt,out,pad", [(BF, F32, 0), (BF, BF, 8), (HF, F32, 16), (HF, HF, 8)])
 def test_ring_gemm(hiplib, rng, m, n, k, dt, out, pad):
     announce(f"ring gemm {m}x{n}x{k} {dt}->{out} pad {pad}")

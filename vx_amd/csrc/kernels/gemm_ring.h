@@ -1,6 +1,6 @@
 /*
- * gemm_ring.h -- launcher of the 128x128-tile GEMM (gemm_ring.hip) and the
- * choice of its splits. Plain host arithmetic.
+ * gemm_ring.h -- launcher of the 128x128- and 256x128-tile GEMM (gemm_ring.hip)
+ * and the choice of its tile and splits. Plain host arithmetic.
  */
 #ifndef VX_AMD_GEMM_RING_H
 #define VX_AMD_GEMM_RING_H
@@ -38,6 +38,18 @@ inline double us(int64_t m, int64_t n, int64_t k, int splits, int cus) {
     t += 3.0 + (double)units * kTile * kTile * 8 / 5e6;
   }
   return t;
+}
+
+/* Whether an undivided launch takes tiles of 256x128, one workgroup to a CU:
+ * where CUs would have two of 128x128 and these fit one to each. They read B
+ * half as often, which counts when it comes from HBM. New inputs each pass,
+ * bf16: 512 x 11008 x 4096 91 -> 79 us (the same ones again 70 -> 66), 1024 x
+ * 5120 x 4096 91 -> 75, 300 x 12288 x 4096 85 -> 70, 512 x 11008 x 2048 50 ->
+ * 44 (the same ones 36 -> 37). Shorter K keeps the smaller tiles: x 1024 30 ->
+ * 28 (22 -> 23), x 256 13.7 -> 14.4. */
+inline bool tall(int64_t m, int64_t n, int64_t k, int cus) {
+  return tiles(m, n) > cus && (m + 2 * kTile - 1) / (2 * kTile) * ((n + kTile - 1) / kTile) <= cus &&
+         k >= 2048;
 }
 
 /* Splits of least time by that model. */

@@ -1,9 +1,10 @@
 /*
- * gemm_ring.hip -- 16-bit GEMMs on 128x128 tiles, for grids that leave many
- * CUs without one of gemm.hip's 256x256 tiles.
+ * gemm_ring.hip -- 16-bit GEMMs on 128x128 or 256x128 tiles, for grids that
+ * leave many CUs without one of gemm.hip's 256x256 tiles.
  *
- * Four waves of 64x64 on v_mfma_f32_16x16x32, two workgroups to a CU. K in
- * stages of 32 through a five-slot LDS ring of buffer-to-LDS loads in the
+ * Waves of 64x64 on v_mfma_f32_16x16x32: four, two workgroups to a CU, or
+ * eight, one to a CU (ring::tall). K in stages of 32 through an LDS ring (five
+ * slots, or six) of buffer-to-LDS loads in the
  * layouts of the ping-pong kernel; a wave reads the next stage's operands
  * while it multiplies this one's, one barrier a stage. With `splits` > 1
  * several workgroups divide a tile's K: each leaves its sums in a workspace
@@ -13,11 +14,12 @@
  * A stage takes 0.34 us where a CU has one workgroup and 0.53 where it has
  * two (690 TFLOP/s at 1024 x 4096 x 4096); what bounds it is getting 16 KiB a
  * stage and workgroup through L1 from L2 (the TCP waits 38% of the cycles,
- * the matrix cores work 41%, the LDS reads take a fifth). Tiles of 128x192
- * (one workgroup to a CU) gave 67.5 us at 512 x 11008 x 4096 and 61 at 1024 x
- * 4096 x 4096 against 70.7 and 49; 256x128 78.8 and 70. Against the kernels
- * that took these shapes: 512 x 11008 x 4096 98 -> 69 us, 1024 x 4096 x 4096 66
- * -> 50, 2048^3 41 -> 28, 512 x 4096 x 11008 in 4 splits 77 -> 61 (in 1: 119).
+ * the matrix cores work 41%, the LDS reads take a fifth); for 256x128, 24 KiB
+ * and 0.47 us, or 0.57 with B from HBM. With four waves the larger tiles leave
+ * the loads' latency open: 128x192 gave 67.5 us at 512 x 11008 x 4096 and 61 at
+ * 1024 x 4096 x 4096 against 70.7 and 49, 256x128 78.8 and 70. Against the kernels
+ * that took these shapes: 512 x 11008 x 4096 102 -> 76 us with
+ * new inputs each pass (98 -> 66 on the same ones), 1024 x 4096 x 4096 66 -> 50, 2048^3 41 -> 28, 512 x 4096 x 11008 in 4 splits 77 -> 61 (in 1: 119).
  */
 #include "../../../include/vx_hardware_runtime.h"
 #include "../vx_hip_common.h"
@@ -32,15 +34,11 @@ namespace {
 
 typedef short i16x4 __attribute__((ext_vector_type(4)));
 
-constexpr int kThreads = 256;
 constexpr int kKs = 32; /* of k per stage */
-constexpr int kBM = ring::kTile, kBN = ring::kTile;
-constexpr int kNS = 5;                                    /* slots: 80 KiB, half of the LDS */
-constexpr int kTM = 4, kTN = 4;                           /* 16x16 blocks of a wave */
-constexpr int kUA = kBM * 4, kUB = kBN * 4;               /* 16-byte units per stage */
-constexpr int kLA = kUA / kThreads, kLB = kUB / kThreads; /* loads per wave */
-constexpr int kRowB = kBN / 8;                            /* units per row of B */
-constexpr int kPart = kBM * kBN * 4;                      /* bytes of a tile's sums */
+constexpr int kBN = ring::kTile;
+constexpr int kTM = 4, kTN = 4;  /* 16x16 blocks of a wave */
+constexpr int kUB = kBN * 4;     /* 16-byte units per stage */
+constexpr int kRowB = kBN / 8;   /* units per row of B */
 
 template <int kOut> __device__ __forceinline__ void put4(void *c, int64_t at, f32x4 v, bool vec) {
   if constexpr (kOut == VX_DTYPE_F32) {
@@ -71,11 +69,16 @@ template <int kOut> __device__ __forceinline__ void put4(void *c, int64_t at, f3
   }
 }
 
-template <bool kBf16, int kOut>
-__global__ __launch_bounds__(kThreads, 2) void gemm_ring(
+template <bool kBf16, int kOut, int kBM>
+__global__ __launch_bounds__(2 * kBM, 2) void gemm_ring(
     const uint16_t *__restrict__ A, const uint16_t *__restrict__ B, void *__restrict__ C,
     int64_t M, int64_t N, int K, int64_t lda, int64_t ldb, int64_t ldc, int tiles_m,
     int tiles_n, int splits, char *__restrict__ ws) {
+  constexpr int kThreads = 2 * kBM;                         /* a wave per 64x64 */
+  constexpr int kNS = kBM == 128 ? 5 : 6;                   /* slots: 80 KiB, or 144 */
+  constexpr int kUA = kBM * 4;                              /* 16-byte units per stage */
+  constexpr int kLA = kUA / kThreads, kLB = kUB / kThreads; /* loads per wave */
+  constexpr int kPart = kBM * kBN * 4;                      /* bytes of a tile's sums */
   __shared__ u32x4 ring[kNS][kUA + kUB];
 
   const int lane = threadIdx.x & 63;
@@ -210,7 +213,7 @@ __global__ __launch_bounds__(kThreads, 2) void gemm_ring(
     multiply(f0);
   }
 
-  if (splits > 1) {
+  if (kBM == ring::kTile && splits > 1) {
     const __amdgpu_buffer_rsrc_t wr = __builtin_amdgcn_make_buffer_rsrc(
         (void *)(ws + ring::kTicketBytes + (int64_t)id * splits * kPart), (short)0,
         splits * kPart, 0x00020000);
@@ -276,12 +279,21 @@ __global__ __launch_bounds__(kThreads, 2) void gemm_ring(
   }
 }
 
+template <bool kBf16, int kOut, int kBM>
+void launch_rows(const GemmArgs &g, int splits, char *ws, hipStream_t s) {
+  const int tiles_m = (int)((g.m + kBM - 1) / kBM), tiles_n = (int)((g.n + kBN - 1) / kBN);
+  hipLaunchKernelGGL((gemm_ring<kBf16, kOut, kBM>), dim3(tiles_m * tiles_n * splits),
+                     dim3(2 * kBM), 0, s, static_cast<const uint16_t *>(g.a), static_cast<const uint16_t *>(g.b),
+                     g.c, g.m, g.n, (int)g.k, g.lda, g.ldb, g.ldc, tiles_m, tiles_n, splits, ws);
+}
+
 template <bool kBf16, int kOut>
 void launch(const GemmArgs &g, int splits, char *ws, hipStream_t s) {
-  const int tiles_m = (int)((g.m + kBM - 1) / kBM), tiles_n = (int)((g.n + kBN - 1) / kBN);
-  hipLaunchKernelGGL((gemm_ring<kBf16, kOut>), dim3(tiles_m * tiles_n * splits), dim3(kThreads), 0,
-                     s, static_cast<const uint16_t *>(g.a), static_cast<const uint16_t *>(g.b),
-                     g.c, g.m, g.n, (int)g.k, g.lda, g.ldb, g.ldc, tiles_m, tiles_n, splits, ws);
+  if (splits == 1 && ring::tall(g.m, g.n, g.k, device_cu_count())) {
+    launch_rows<kBf16, kOut, 2 * ring::kTile>(g, 1, nullptr, s);
+  } else {
+    launch_rows<kBf16, kOut, ring::kTile>(g, splits, ws, s);
+  }
 }
 
 } // namespace
