@@ -124,3 +124,22 @@ def test_infinities_and_nans(hiplib, rng):
     ok = np.isfinite(want)
     assert np.max(np.abs(c - want)[ok] / np.abs(want)[ok]) < (k + 2) * 2.0 ** -24
     assert np.isnan(c[3, 7]) and np.isnan(c[3, 150]) and np.isposinf(c[3, 0])
+
+
+@pytest.mark.parametrize("k", [140, 3000])  # in one workgroup a tile, and divided
+@pytest.mark.parametrize("exponent", [-101, -112, -124, -134, -140])
+def test_tiny_elements_of_ordinary_rows(hiplib, rng, k, exponent):
+    """Rows that hold ordinary values opposite zeros and tiny ones opposite
+    large ones: each sum is of the tiny ones' products alone."""
+    announce(f"f32 gemm, elements of 2^{exponent} in ordinary rows, k {k}")
+    m, n = 150, 140
+    a = rng.uniform(1, 2, (m, k)) * rng.choice([-1, 1], (m, k))
+    b = rng.uniform(1, 2, (k, n)) * rng.choice([-1, 1], (k, n))
+    a, b = a.astype(np.float32), b.astype(np.float32)
+    tiny = rng.choice(k, 5, replace=False)
+    a[17, tiny] *= np.float32(2.0 ** exponent)
+    b[:, 99] = 0
+    b[tiny, 99] = (rng.uniform(1, 2, 5) * 2.0 ** 120).astype(np.float32)
+    check(product(hiplib, a, b), a, b)
+    at, bt = np.ascontiguousarray(a.T), np.ascontiguousarray(b.T)
+    check(product(hiplib, bt, at), bt, at)

@@ -12,10 +12,10 @@ namespace f32 {
 
 constexpr int kTile = 128;
 /* A split launch's workspace: a ticket per tile, zero between launches, then
- * each split's sums and magnitudes. */
+ * each split's sums. */
 constexpr int kMaxSplitTiles = 1024;
 constexpr int64_t kTicketBytes = kMaxSplitTiles * 4;
-constexpr int kPart = (kTile * kTile + 2 * kTile) * 4;
+constexpr int kPart = kTile * kTile * 4;
 
 inline int64_t tiles(int64_t m, int64_t n) {
   return ((m + kTile - 1) / kTile) * ((n + kTile - 1) / kTile);

@@ -4,13 +4,17 @@
  *
  * An f32 value is the exact sum of three bf16 values, its 24 significant bits
  * 8 at a time, and the product of two such values is exact in f32. Of the nine
- * products of a pair the six of up to 2^-16 of the largest are added (the rest
- * are below 2^-24 of it, under the rounding of the f32 sums): the large ones
- * in one accumulator, the other five in a second, added at the end. Six
- * v_mfma_f32_16x16x32_bf16 do 32 of k in 96 cycles; f32 MFMAs take 256.
- * Infinities, and rows of A or columns of B without a value of 2^-100 or
- * more, whose last bits bf16 cannot hold, are left to f32 MFMAs: a tile that
- * met one is computed again that way. (A NaN passes through the planes.)
+ * products of a pair the six largest are added: the first in one accumulator,
+ * the other five in a second, added at the end.
+ * Six v_mfma_f32_16x16x32_bf16 do 32 of k in 96 cycles; f32 MFMAs take 256.
+ *
+ * What bf16 cannot hold is left to f32 MFMAs: a block of 16 x 16 sums is
+ * computed again that way, over the workgroup's k, where one of them is not
+ * finite or lies below 2^-100, or where an element below 2^-100 may have lost
+ * bits that count in it. The last needs, of each row and column, the greatest
+ * magnitude and whether it has such an element; a tile that met one reads its
+ * operands again for them (2048^3 with a third of A below 2^-110 124 us, with
+ * an infinity in every tile 154, against 248 where all is done in f32).
  *
  * 128 x 128 tiles, eight waves of 64 x 32, K in stages of 32 through two LDS
  * slots. A thread loads 8 k of one row of A and of one column of B, splits
@@ -40,13 +44,13 @@
 namespace vxk {
 namespace {
 
-typedef float f32x16 __attribute__((ext_vector_type(16)));
-
 constexpr int kThreads = 512;
 constexpr int kTile = f32::kTile;
 constexpr int kKs = 32;               /* of k per stage */
 constexpr int kPlane = kTile * 4;     /* 16-byte units */
+constexpr int kRows32 = kTile * 8;    /* of a stage's rows in f32 */
 constexpr float kLeast = 7.888609052210118e-31f; /* 2^-100 */
+constexpr uint32_t kLeastBits = (127 - 100) << 23;
 
 struct __attribute__((packed, aligned(4))) Four {
   f32x4 v;
@@ -57,6 +61,8 @@ struct Regs {
 };
 
 __device__ __forceinline__ int unit(int row, int c) { return row * 4 + (c ^ ((row >> 1) & 3)); }
+/* The same in f32, a chunk being 4 k. */
+__device__ __forceinline__ int unit32(int row, int c) { return row * 8 + (c ^ (row & 7)); }
 
 /* Eight values as the three planes' 16 bytes. */
 __device__ __forceinline__ void split8(const float (&x)[8], u32x4 (&p)[3]) {
@@ -80,7 +86,8 @@ __global__ __launch_bounds__(kThreads, 2) void gemm_f32_mfma(
     const float *__restrict__ A, const float *__restrict__ B, float *__restrict__ C, int64_t M,
     int64_t N, int64_t K, int64_t lda, int64_t ldb, int64_t ldc, int tiles_m, int tiles_n,
     int splits, char *__restrict__ ws) {
-  __shared__ u32x4 lds[2][2][3][kPlane]; /* [slot][A, B][plane] */
+  /* [slot][A, B][plane][kPlane]; in f32 [slot][A, B][kRows32] */
+  __shared__ u32x4 lds[2 * 2 * 3 * kPlane];
   const int t = threadIdx.x;
   const int lane = t & 63;
   const int wave = __builtin_amdgcn_readfirstlane(t >> 6);
@@ -134,68 +141,6 @@ __global__ __launch_bounds__(kThreads, 2) void gemm_f32_mfma(
       r.b[e] = st * kKs + 8 * b_chunk + e < left ? (b + e * ldb)[b_off] : 0.0f;
     }
   };
-  float a_max = 0.0f, b_max = 0.0f; /* of the row's and column's magnitudes */
-  auto stash = [&](const Regs &r, int slot) {
-    u32x4 p[3];
-#pragma unroll
-    for (int e = 0; e < 8; ++e) {
-      a_max = fmaxf(a_max, __builtin_fabsf(r.a[e]));
-      b_max = fmaxf(b_max, __builtin_fabsf(r.b[e]));
-    }
-    split8(r.a, p);
-#pragma unroll
-    for (int i = 0; i < 3; ++i) {
-      lds[slot][0][i][unit(a_row, a_chunk)] = p[i];
-    }
-    split8(r.b, p);
-#pragma unroll
-    for (int i = 0; i < 3; ++i) {
-      lds[slot][1][i][unit(b_col, b_chunk)] = p[i];
-    }
-  };
-
-  /* hi, lo[i][j]: rows 64 wm + 16 i + l16, columns 32 wn + 16 j + 4 g .. + 3 */
-  f32x4 hi[4][2], lo[4][2];
-#pragma unroll
-  for (int i = 0; i < 4; ++i) {
-#pragma unroll
-    for (int j = 0; j < 2; ++j) {
-      hi[i][j] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
-      lo[i][j] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
-    }
-  }
-  u32x4 af[3][4], bf[3][2];
-  auto fragments = [&](int slot) {
-#pragma unroll
-    for (int p = 0; p < 3; ++p) {
-#pragma unroll
-      for (int j = 0; j < 2; ++j) {
-        bf[p][j] = lds[slot][1][p][unit(32 * wn + 16 * j + l16, g)];
-      }
-#pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        af[p][i] = lds[slot][0][p][unit(64 * wm + 16 * i + l16, g)];
-      }
-    }
-  };
-  auto multiply = [&]() {
-    auto add = [&](int pa_, int pb_, f32x4 (&c)[4][2]) {
-#pragma unroll
-      for (int j = 0; j < 2; ++j) {
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-          c[i][j] = mfma16<true>(bf[pb_][j], af[pa_][i], c[i][j]);
-        }
-      }
-    };
-    add(0, 0, hi);
-    add(0, 1, lo);
-    add(1, 0, lo);
-    add(1, 1, lo);
-    add(0, 2, lo);
-    add(2, 0, lo);
-  };
-
   auto load_any = [&](Regs &r, int64_t st) {
     if (st < whole) {
       load(r, st);
@@ -203,6 +148,139 @@ __global__ __launch_bounds__(kThreads, 2) void gemm_f32_mfma(
       load_last(r, st);
     }
   };
+
+  /* c[i][j]: rows 64 wm + 16 i + l16, columns 32 wn + 16 j + 4 g .. + 3 */
+  f32x4 c[4][2];
+
+  /* The blocks of c whose bit 2 i + j is set, over the workgroup's k, on
+   * v_mfma_f32_16x16x4_f32. Step e of a 16-k half takes k = 4 g + e of it from
+   * lane group g, on both sides, so an operand is four steps' 16 bytes. */
+  auto in_f32 = [&](uint32_t blocks) {
+    auto stash = [&](const Regs &r, int slot) {
+#pragma unroll
+      for (int h = 0; h < 2; ++h) {
+        lds[2 * slot * kRows32 + unit32(a_row, 2 * a_chunk + h)] = __builtin_bit_cast(
+            u32x4, f32x4{r.a[4 * h], r.a[4 * h + 1], r.a[4 * h + 2], r.a[4 * h + 3]});
+        lds[(2 * slot + 1) * kRows32 + unit32(b_col, 2 * b_chunk + h)] = __builtin_bit_cast(
+            u32x4, f32x4{r.b[4 * h], r.b[4 * h + 1], r.b[4 * h + 2], r.b[4 * h + 3]});
+      }
+    };
+#pragma unroll
+    for (int q = 0; q < 8; ++q) {
+      if (blocks >> q & 1) {
+        c[q >> 1][q & 1] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+      }
+    }
+    Regs r;
+    load_any(r, 0);
+    stash(r, 0);
+    if (stages > 1) {
+      load_any(r, 1);
+    }
+    lds_barrier();
+    for (int64_t st = 0; st < stages; ++st) {
+      const int slot = (int)(st & 1);
+      if (st + 1 < stages) {
+        stash(r, slot ^ 1);
+      }
+      if (st + 2 < stages) {
+        load_any(r, st + 2);
+      }
+#pragma unroll
+      for (int h = 0; h < 2; ++h) {
+        if (st * kKs + 16 * h < left) {
+          f32x4 af[4], bf[2];
+#pragma unroll
+          for (int i = 0; i < 4; ++i) {
+            af[i] = __builtin_bit_cast(
+                f32x4, lds[2 * slot * kRows32 + unit32(64 * wm + 16 * i + l16, 4 * h + g)]);
+          }
+#pragma unroll
+          for (int j = 0; j < 2; ++j) {
+            bf[j] = __builtin_bit_cast(
+                f32x4, lds[(2 * slot + 1) * kRows32 + unit32(32 * wn + 16 * j + l16, 4 * h + g)]);
+          }
+#pragma unroll
+          for (int i = 0; i < 4; ++i) {
+#pragma unroll
+            for (int j = 0; j < 2; ++j) {
+              if (blocks >> (2 * i + j) & 1) {
+#pragma unroll
+                for (int e = 0; e < 4; ++e) {
+                  c[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(bf[j][e], af[i][e], c[i][j], 0, 0, 0);
+                }
+              }
+            }
+          }
+        }
+      }
+      lds_barrier();
+    }
+  };
+
+  __shared__ int again;
+  if (t == 0) {
+    again = 0;
+  }
+  /* The least magnitude but zero, as its bits times two, less one. */
+  constexpr uint32_t kTiny = 2 * kLeastBits - 1;
+  uint32_t least = ~0u;
+  auto stash = [&](const Regs &r, int slot) {
+    u32x4 p[3];
+#pragma unroll
+    for (int e = 0; e < 8; ++e) {
+      least = min(least, 2 * __float_as_uint(r.a[e]) - 1);
+      least = min(least, 2 * __float_as_uint(r.b[e]) - 1);
+    }
+    split8(r.a, p);
+#pragma unroll
+    for (int i = 0; i < 3; ++i) {
+      lds[(6 * slot + i) * kPlane + unit(a_row, a_chunk)] = p[i];
+    }
+    split8(r.b, p);
+#pragma unroll
+    for (int i = 0; i < 3; ++i) {
+      lds[(6 * slot + 3 + i) * kPlane + unit(b_col, b_chunk)] = p[i];
+    }
+  };
+  f32x4 lo[4][2];
+#pragma unroll
+  for (int q = 0; q < 8; ++q) {
+    c[q >> 1][q & 1] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+    lo[q >> 1][q & 1] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+  }
+  u32x4 af[3][4], bf[3][2];
+  auto fragments = [&](int slot) {
+#pragma unroll
+    for (int p = 0; p < 3; ++p) {
+#pragma unroll
+      for (int j = 0; j < 2; ++j) {
+        bf[p][j] = lds[(6 * slot + 3 + p) * kPlane + unit(32 * wn + 16 * j + l16, g)];
+      }
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        af[p][i] = lds[(6 * slot + p) * kPlane + unit(64 * wm + 16 * i + l16, g)];
+      }
+    }
+  };
+  auto multiply = [&]() {
+    auto add = [&](int pa_, int pb_, f32x4 (&x)[4][2]) {
+#pragma unroll
+      for (int j = 0; j < 2; ++j) {
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          x[i][j] = mfma16<true>(bf[pb_][j], af[pa_][i], x[i][j]);
+        }
+      }
+    };
+    add(0, 0, c);
+    add(0, 1, lo);
+    add(1, 0, lo);
+    add(1, 1, lo);
+    add(0, 2, lo);
+    add(2, 0, lo);
+  };
+
   /* Entering stage s: it is in slot s % 2, the next in r[(s + 1) % 3], the one
    * after in r[(s + 2) % 3]. */
   Regs r[3];
@@ -224,7 +302,7 @@ __global__ __launch_bounds__(kThreads, 2) void gemm_f32_mfma(
 #pragma unroll
     for (int i = 0; i < 48; ++i) {
       __builtin_amdgcn_sched_group_barrier(0x008, 1, 0); /* MFMA */
-      __builtin_amdgcn_sched_group_barrier(0x002, 3, 0); /* VALU */
+      __builtin_amdgcn_sched_group_barrier(0x002, 4, 0); /* VALU */
     }
     lds_barrier();
   };
@@ -248,56 +326,113 @@ __global__ __launch_bounds__(kThreads, 2) void gemm_f32_mfma(
     lds_barrier();
   }
 
-  /* The row's other three threads are its lane's neighbours, the column's
-   * other three in other waves. */
-  auto odd = [&](float v) { return !(v < INFINITY) || (v > 0.0f && v < kLeast); };
+  uint32_t small = least, large = 0; /* of the sums, likewise, and the greatest */
 #pragma unroll
-  for (int o = 1; o < 4; o *= 2) {
-    a_max = fmaxf(a_max, __shfl_xor(a_max, o));
-  }
-  float *cols = reinterpret_cast<float *>(&lds[0][0][0][0]); /* [4][128] */
-  cols[b_chunk * kTile + b_col] = b_max;
-  __syncthreads();
+  for (int q = 0; q < 8; ++q) {
 #pragma unroll
-  for (int c = 0; c < 4; ++c) {
-    b_max = fmaxf(b_max, cols[c * kTile + b_col]);
-  }
-#pragma unroll
-  for (int i = 0; i < 4; ++i) {
-#pragma unroll
-    for (int j = 0; j < 2; ++j) {
-#pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        hi[i][j][e] = hi[i][j][e] + lo[i][j][e];
-      }
+    for (int e = 0; e < 4; ++e) {
+      const float v = c[q >> 1][q & 1][e] + lo[q >> 1][q & 1][e];
+      c[q >> 1][q & 1][e] = v;
+      small = min(small, 2 * __float_as_uint(v) - 1);
+      large = max(large, __float_as_uint(v) & 0x7fffffffu);
     }
   }
+  if (small < kTiny || large >= 0x7f800000u) {
+    again = 1;
+  }
+  __syncthreads();
+  if (again) {
+    /* Blocks of c to compute again (bit 2 i + j): sums that are not finite,
+     * or too small for the planes' products. */
+    uint32_t odd = 0;
+#pragma unroll
+    for (int q = 0; q < 8; ++q) {
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        const float v = __builtin_fabsf(c[q >> 1][q & 1][e]);
+        odd |= (uint32_t)(!(v < INFINITY) || (v > 0.0f && v < kLeast)) << q;
+      }
+    }
+    if (__syncthreads_or(least < kTiny)) {
+      /* What such values may have lost, at most 2^-126 of each, against the
+       * result: the rows' and columns' greatest and least are read again. */
+      float a_max = 0.0f, b_max = 0.0f;
+      uint32_t a_min = ~0u, b_min = ~0u;
+      for (st = 0; st < stages; st += 3) {
+#pragma unroll
+        for (int i = 0; i < 3; ++i) {
+          load_any(r[i], min(st + i, stages - 1));
+        }
+#pragma unroll
+        for (int i = 0; i < 3; ++i) {
+#pragma unroll
+          for (int e = 0; e < 8; ++e) {
+            a_max = fmaxf(a_max, __builtin_fabsf(r[i].a[e]));
+            b_max = fmaxf(b_max, __builtin_fabsf(r[i].b[e]));
+            a_min = min(a_min, 2 * __float_as_uint(r[i].a[e]) - 1);
+            b_min = min(b_min, 2 * __float_as_uint(r[i].b[e]) - 1);
+          }
+        }
+      }
+      struct Side {
+        float most, tiny; /* `tiny`: whether there is one, 1 or 0 */
+      };
+      Side *rows = reinterpret_cast<Side *>(&lds[0]); /* [4][128] each */
+      Side *cols = rows + 4 * kTile;
+      rows[a_chunk * kTile + a_row] = Side{a_max, a_min < kTiny ? 1.0f : 0.0f};
+      cols[b_chunk * kTile + b_col] = Side{b_max, b_min < kTiny ? 1.0f : 0.0f};
+      __syncthreads();
+      auto side = [&](const Side *of, int at) {
+        Side x = of[at];
+#pragma unroll
+        for (int q = 1; q < 4; ++q) {
+          x.most = fmaxf(x.most, of[q * kTile + at].most);
+          x.tiny = fmaxf(x.tiny, of[q * kTile + at].tiny);
+        }
+        return x;
+      };
+      const float lost = (float)(stages * kKs) * (kLeast * 2.0f);
+#pragma unroll
+      for (int j = 0; j < 2; ++j) {
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          const Side b = side(cols, 32 * wn + 16 * j + 4 * g + e);
+#pragma unroll
+          for (int i = 0; i < 4; ++i) {
+            const Side a = side(rows, 64 * wm + 16 * i + l16);
+            odd |= (uint32_t)(lost * (a.tiny * b.most + b.tiny * a.most) >
+                              __builtin_fabsf(c[i][j][e]))
+                   << (2 * i + j);
+          }
+        }
+      }
+    }
+    uint32_t blocks = 0; /* of the wave */
+#pragma unroll
+    for (int q = 0; q < 8; ++q) {
+      blocks |= (uint32_t)(__builtin_amdgcn_ballot_w64((odd >> q & 1) != 0) != 0) << q;
+    }
+    if (__syncthreads_or(blocks != 0)) {
+      in_f32(blocks);
+    }
+  }
+
   if (splits > 1) {
-    /* The sums, then the magnitudes, go past the caches that other XCDs do not
-     * see; the workgroup with the last ticket adds all of them up in order. */
+    /* The sums go past the caches that other XCDs do not see; the workgroup
+     * with the last ticket adds all of them up in order. */
     const __amdgpu_buffer_rsrc_t wr = __builtin_amdgcn_make_buffer_rsrc(
         (void *)(ws + f32::kTicketBytes + (int64_t)id * splits * f32::kPart), (short)0,
         splits * f32::kPart, 0x00020000);
-    constexpr int kMax = kTile * kTile * 4; /* [128] of the rows, [128] of the columns */
     const int at = t * 16;
     __shared__ int last;
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
 #pragma unroll
       for (int j = 0; j < 2; ++j) {
-        __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, hi[i][j]), wr,
+        __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, c[i][j]), wr,
                                                at + (2 * i + j) * kThreads * 16,
                                                split * f32::kPart, 16 /* sc1 */);
       }
-    }
-    if (a_chunk == 0) {
-      __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(a_max), wr, kMax + a_row * 4,
-                                            split * f32::kPart, 16 /* sc1 */);
-    }
-    if (b_chunk == 0) {
-      __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(b_max), wr,
-                                            kMax + (kTile + b_col) * 4, split * f32::kPart,
-                                            16 /* sc1 */);
     }
     __builtin_amdgcn_s_waitcnt(0);
     __syncthreads();
@@ -313,7 +448,6 @@ __global__ __launch_bounds__(kThreads, 2) void gemm_f32_mfma(
     if (!last) {
       return;
     }
-    a_max = b_max = 0.0f;
     for (int s = 0; s < splits; ++s) {
       f32x4 v[4][2];
 #pragma unroll
@@ -325,92 +459,33 @@ __global__ __launch_bounds__(kThreads, 2) void gemm_f32_mfma(
                                                   s * f32::kPart, 16 /* sc1 */));
         }
       }
-      a_max = fmaxf(a_max, __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(
-                               wr, kMax + a_row * 4, s * f32::kPart, 16 /* sc1 */)));
-      b_max = fmaxf(b_max, __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(
-                               wr, kMax + (kTile + b_col) * 4, s * f32::kPart, 16 /* sc1 */)));
 #pragma unroll
       for (int i = 0; i < 4; ++i) {
 #pragma unroll
         for (int j = 0; j < 2; ++j) {
-          hi[i][j] = s == 0 ? v[i][j] : hi[i][j] + v[i][j];
+          c[i][j] = s == 0 ? v[i][j] : c[i][j] + v[i][j];
         }
       }
     }
   }
-  if (!__syncthreads_or(odd(a_max) || odd(b_max))) {
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
+  for (int i = 0; i < 4; ++i) {
 #pragma unroll
-      for (int j = 0; j < 2; ++j) {
-        const int64_t row = m0 + 64 * wm + 16 * i + l16;
-        const int64_t col = n0 + 32 * wn + 16 * j + 4 * g;
-        if (row < M && col < N) {
-          float *c = C + row * ldc + col;
-          if (col + 3 < N) {
-            reinterpret_cast<Four *>(c)->v = hi[i][j];
-          } else {
+    for (int j = 0; j < 2; ++j) {
+      const int64_t row = m0 + 64 * wm + 16 * i + l16;
+      const int64_t col = n0 + 32 * wn + 16 * j + 4 * g;
+      if (row < M && col < N) {
+        float *p = C + row * ldc + col;
+        if (col + 3 < N) {
+          reinterpret_cast<Four *>(p)->v = c[i][j];
+        } else {
 #pragma unroll
-            for (int e = 0; e < 3; ++e) {
-              if (col + e < N) {
-                c[e] = hi[i][j][e];
-              }
+          for (int e = 0; e < 3; ++e) {
+            if (col + e < N) {
+              p[e] = c[i][j][e];
             }
           }
         }
-      }
-    }
-    return;
-  }
-
-  /* The tile again on v_mfma_f32_32x32x2_f32: stages of 16 of k through one
-   * LDS slot, operands as [k][m] and [k][n] with 32 floats between the two
-   * half-waves' rows. */
-  constexpr int kFs = 16, kPad = kTile + 32;
-  float(*as)[kPad] = reinterpret_cast<float(*)[kPad]>(&lds[0][0][0][0]);
-  float(*bs)[kPad] = as + kFs;
-  f32x16 acc[2];
-#pragma unroll
-  for (int i = 0; i < 2; ++i) {
-#pragma unroll
-    for (int r = 0; r < 16; ++r) {
-      acc[i][r] = 0.0f;
-    }
-  }
-  const int64_t am = min(m0 + (t >> 2), M - 1), bn0 = n0 + 4 * (t & 31);
-  const int ak = 4 * (t & 3), bk = t >> 5;
-  for (int64_t k0 = 0; k0 < K; k0 += kFs) {
-    float ra[4], rb[4];
-#pragma unroll
-    for (int e = 0; e < 4; ++e) {
-      ra[e] = k0 + ak + e < K ? A[am * lda + k0 + ak + e] : 0.0f;
-      rb[e] = k0 + bk < K ? B[(k0 + bk) * ldb + min(bn0 + e, N - 1)] : 0.0f;
-    }
-    __syncthreads();
-#pragma unroll
-    for (int e = 0; e < 4; ++e) {
-      as[ak + e][t >> 2] = ra[e];
-      bs[bk][4 * (t & 31) + e] = rb[e];
-    }
-    __syncthreads();
-#pragma unroll
-    for (int kk = 0; kk < kFs; kk += 2) {
-      const float b = bs[kk + (lane >> 5)][32 * wn + (lane & 31)];
-#pragma unroll
-      for (int i = 0; i < 2; ++i) {
-        const float a = as[kk + (lane >> 5)][64 * wm + 32 * i + (lane & 31)];
-        acc[i] = __builtin_amdgcn_mfma_f32_32x32x2f32(a, b, acc[i], 0, 0, 0);
-      }
-    }
-  }
-#pragma unroll
-  for (int i = 0; i < 2; ++i) {
-    const int64_t col = n0 + 32 * wn + (lane & 31);
-#pragma unroll
-    for (int r = 0; r < 16; ++r) {
-      const int64_t row = m0 + 64 * wm + 32 * i + 8 * (r >> 2) + 4 * (lane >> 5) + (r & 3);
-      if (row < M && col < N) {
-        C[row * ldc + col] = acc[i][r];
       }
     }
   }
