@@ -143,3 +143,20 @@ def test_tiny_elements_of_ordinary_rows(hiplib, rng, k, exponent):
     check(product(hiplib, a, b), a, b)
     at, bt = np.ascontiguousarray(a.T), np.ascontiguousarray(b.T)
     check(product(hiplib, bt, at), bt, at)
+
+
+@pytest.mark.parametrize("k", [1, 31, 128, 140, 2100])
+def test_single_products(hiplib, rng, k):
+    """One value in each row of A: every sum is one product, whose error is
+    its rounding (2^-24) and the products of planes left out (2^-24, of values
+    whose planes are worst the most)."""
+    announce(f"f32 gemm, single products, k {k}")
+    m, n = 140, 150
+    a = np.zeros((m, k), np.float32)
+    values = np.float32(1 + 2.0 ** -7 - 2.0 ** -23) * rng.choice([1, -1], m)
+    values[m // 2:] = rng.uniform(1, 2, m - m // 2)
+    a[np.arange(m), rng.integers(0, k, m)] = values
+    b = np.full((k, n), 1 + 2.0 ** -7 - 2.0 ** -23, np.float32)
+    b[:, n // 2:] = rng.uniform(1, 2, (k, n - n // 2))
+    want = a.astype(np.float64) @ b.astype(np.float64)
+    assert np.max(np.abs(product(hiplib, a, b) - want) / np.abs(want)) <= 2.1 * 2.0 ** -24

@@ -2,10 +2,12 @@
  * gemm_f32.hip -- f32 GEMM for products large enough that the exact-order
  * kernel's rate matters, on bf16 MFMAs.
  *
- * An f32 value is the exact sum of three bf16 values, its 24 significant bits
- * 8 at a time, and the product of two such values is exact in f32. Of the nine
- * products of a pair the six largest are added: the first in one accumulator,
- * the other five in a second, added at the end.
+ * An f32 value is the exact sum of three bf16 values, each the rest of the one
+ * before rounded to nearest, and the product of two such values is exact in
+ * f32. Of the nine products of a pair the six largest are added: the first in
+ * one accumulator, the other five in a second, added at the end. The rounded
+ * rests are at most 2^-8 and 2^-17 of the value's leading bit, so that what is
+ * left out is at most 2^-24 of the product, of either sign.
  * Six v_mfma_f32_16x16x32_bf16 do 32 of k in 96 cycles; f32 MFMAs take 256.
  *
  * What bf16 cannot hold is left to f32 MFMAs: a block of 16 x 16 sums is
@@ -64,21 +66,25 @@ __device__ __forceinline__ int unit(int row, int c) { return row * 4 + (c ^ ((ro
 /* The same in f32, a chunk being 4 k. */
 __device__ __forceinline__ int unit32(int row, int c) { return row * 8 + (c ^ (row & 7)); }
 
+/* Two values rounded to bf16, the first in the lower half. */
+__device__ __forceinline__ uint32_t round2(float lo, float hi) {
+  typedef float f32x2 __attribute__((ext_vector_type(2)));
+  typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
+  return __builtin_bit_cast(uint32_t, __builtin_convertvector((f32x2{lo, hi}), bf16x2));
+}
+
 /* Eight values as the three planes' 16 bytes. */
 __device__ __forceinline__ void split8(const float (&x)[8], u32x4 (&p)[3]) {
-  uint32_t u[8], r[8], s[8];
 #pragma unroll
-  for (int e = 0; e < 8; ++e) {
-    u[e] = __float_as_uint(x[e]);
-    const float d = x[e] - __uint_as_float(u[e] & 0xffff0000u);
-    r[e] = __float_as_uint(d);
-    s[e] = __float_as_uint(d - __uint_as_float(r[e] & 0xffff0000u));
-  }
+  for (int w = 0; w < 4; ++w) {
+    float lo = x[2 * w], hi = x[2 * w + 1];
 #pragma unroll
-  for (int w = 0; w < 4; ++w) { /* upper halves */
-    p[0][w] = __builtin_amdgcn_perm(u[2 * w + 1], u[2 * w], 0x07060302u);
-    p[1][w] = __builtin_amdgcn_perm(r[2 * w + 1], r[2 * w], 0x07060302u);
-    p[2][w] = __builtin_amdgcn_perm(s[2 * w + 1], s[2 * w], 0x07060302u);
+    for (int i = 0; i < 3; ++i) {
+      const uint32_t r = round2(lo, hi);
+      p[i][w] = r;
+      lo -= __uint_as_float(r << 16);
+      hi -= __uint_as_float(r & 0xffff0000u);
+    }
   }
 }
 
