@@ -1,4 +1,4 @@
-"""The f32 GEMM on bf16 planes (gemm_f32.hip): what its planes cannot hold,
+"""The f32 GEMM on bf16 planes, and on f32 MFMAs (gemm_f32.hip): what its planes cannot hold,
 and the edges of its stages, against the f64 product. The tolerance is the
 bound of f32 sums of products in any order plus what the dropped planes'
 products come to: |C - AB| <= (K + 2) 2^-24 (|A| |B|)."""
@@ -49,7 +49,8 @@ def check(c, a, b):
 
 @pytest.mark.parametrize("m,n,k", [(1, 1, 1), (128, 128, 31), (129, 127, 32), (127, 130, 33), (5, 300, 64),
                                    (300, 5, 95), (256, 384, 96), (130, 131, 129), (200, 200, 1000),
-                                   (130, 131, 2047), (20, 1000, 4100)])
+                                   (130, 131, 2047), (20, 1000, 4100), (1, 1, 127), (130, 131, 128),
+                                   (129, 127, 160), (127, 130, 161), (60, 300, 257), (300, 60, 288), (33, 70, 320)])
 @pytest.mark.parametrize("pad", [0, 1])
 def test_edges_of_stages_and_tiles(hiplib, rng, m, n, k, pad):
     announce(f"f32 gemm {m}x{n}x{k} pad {pad}")
@@ -60,12 +61,13 @@ def test_edges_of_stages_and_tiles(hiplib, rng, m, n, k, pad):
     assert np.array_equal(c, product(hiplib, a, b, pad))
 
 
+@pytest.mark.parametrize("k", [90, 260])  # on f32 MFMAs, and in planes
 @pytest.mark.parametrize("lo,hi,other", [(-60, 60, 0), (-126, -100, 100), (90, 126, -100)])
-def test_magnitudes(hiplib, rng, lo, hi, other):
+def test_magnitudes(hiplib, rng, lo, hi, other, k):
     """Elements of every magnitude f32 has, times ones that keep the products
     inside its range."""
     announce(f"f32 gemm, magnitudes 2^{lo} .. 2^{hi}")
-    m, n, k = 150, 140, 90
+    m, n = 150, 140
 
     def draw(shape, exponents):
         return (rng.uniform(1, 2, shape) * rng.choice([-1, 1], shape) * 2.0 ** exponents).astype(np.float32)
@@ -77,11 +79,12 @@ def test_magnitudes(hiplib, rng, lo, hi, other):
     check(product(hiplib, bt, at), bt, at)
 
 
-def test_rows_and_columns_too_small_for_the_planes(hiplib, rng):
+@pytest.mark.parametrize("k", [100, 330])
+def test_rows_and_columns_too_small_for_the_planes(hiplib, rng, k):
     """A row of A and a column of B of subnormal and other tiny values, next
     to zeros, in tiles of ordinary ones."""
     announce("f32 gemm, tiny rows")
-    m, n, k = 260, 300, 100
+    m, n = 260, 300
     a = rng.uniform(-1, 1, (m, k)).astype(np.float32)
     b = rng.uniform(-1, 1, (k, n)).astype(np.float32)
     a[140] = (rng.uniform(-1, 1, k) * 2.0 ** -120).astype(np.float32)
@@ -108,11 +111,12 @@ def test_tiny_and_infinite_rows_over_splits(hiplib, rng):
     assert np.array_equal(c[199], np.where(b[2500] > 0, np.inf, -np.inf))
 
 
-def test_infinities_and_nans(hiplib, rng):
+@pytest.mark.parametrize("k", [70, 200])
+def test_infinities_and_nans(hiplib, rng, k):
     """As f32 arithmetic has them: an infinity times a finite value is an
     infinity of the product's sign, times zero NaN; nothing else is touched."""
     announce("f32 gemm, infinities and NaNs")
-    m, n, k = 260, 260, 70
+    m, n = 260, 260
     a = rng.uniform(0.5, 1, (m, k)).astype(np.float32)
     b = rng.uniform(0.5, 1, (k, n)).astype(np.float32)
     a[3, 69], a[200, 0], b[5, 150], b[69, 7] = np.inf, np.nan, -np.inf, 0.0

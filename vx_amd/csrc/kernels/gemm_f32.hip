@@ -1,6 +1,6 @@
 /*
  * gemm_f32.hip -- f32 GEMM for products large enough that the exact-order
- * kernel's rate matters, on bf16 MFMAs.
+ * kernel's rate matters, on bf16 MFMAs, or on f32 MFMAs where K is short.
  *
  * An f32 value is the exact sum of three bf16 values, each the rest of the one
  * before rounded to nearest, and the product of two such values is exact in
@@ -30,6 +30,11 @@
  * barriers (taking a SIMD's two waves in turns, one reading while the other
  * multiplies, costs a barrier more and gave the same: 108 us).
  *
+ * K below f32::kPlanesMinK: the same tile on f32 MFMAs throughout, one LDS slot
+ * and three workgroups to a CU, whose loads and stores overlap. Writing C
+ * bounds it. The planes' way there, against it: 8192^2 x 16 103 us, 52; 328 x
+ * 601168 x 8 365, 197; 4096^2 x 64 34, 27.
+ *
  * Against f32 MFMAs in the same tile: 2048^3 248 -> 92 us with new inputs each
  * pass (188 TFLOP/s), 258 -> 104 with the same ones; error against 64 bits
  * 8.1e-7 -> 2.5e-7 at 2048^3, 1.1e-6 -> 3.8e-7 at K = 4096. Grids of fewer
@@ -42,6 +47,7 @@
 #include "gemm_pp_layout.h"
 #include "vx_lds_dma.hip.h"
 #include "vx_mfma16.hip.h"
+#include "vx_wave_ops.hip.h"
 
 namespace vxk {
 namespace {
@@ -88,12 +94,13 @@ __device__ __forceinline__ void split8(const float (&x)[8], u32x4 (&p)[3]) {
   }
 }
 
-__global__ __launch_bounds__(kThreads, 2) void gemm_f32_mfma(
+template <bool kPlanes>
+__global__ __launch_bounds__(kThreads, kPlanes ? 2 : 6) void gemm_f32_mfma(
     const float *__restrict__ A, const float *__restrict__ B, float *__restrict__ C, int64_t M,
     int64_t N, int64_t K, int64_t lda, int64_t ldb, int64_t ldc, int tiles_m, int tiles_n,
     int splits, char *__restrict__ ws) {
-  /* [slot][A, B][plane][kPlane]; in f32 [slot][A, B][kRows32] */
-  __shared__ u32x4 lds[2 * 2 * 3 * kPlane];
+  /* [slot][A, B][plane][kPlane]; in f32 [slot][A, B][kRows32], one slot alone */
+  __shared__ u32x4 lds[kPlanes ? 2 * 2 * 3 * kPlane : 2 * kRows32];
   const int t = threadIdx.x;
   const int lane = t & 63;
   const int wave = __builtin_amdgcn_readfirstlane(t >> 6);
@@ -179,18 +186,28 @@ __global__ __launch_bounds__(kThreads, 2) void gemm_f32_mfma(
     }
     Regs r;
     load_any(r, 0);
-    stash(r, 0);
-    if (stages > 1) {
-      load_any(r, 1);
-    }
-    lds_barrier();
-    for (int64_t st = 0; st < stages; ++st) {
-      const int slot = (int)(st & 1);
-      if (st + 1 < stages) {
-        stash(r, slot ^ 1);
+    if constexpr (kPlanes) {
+      stash(r, 0);
+      if (stages > 1) {
+        load_any(r, 1);
       }
-      if (st + 2 < stages) {
-        load_any(r, st + 2);
+      lds_barrier();
+    }
+    for (int64_t st = 0; st < stages; ++st) {
+      const int slot = kPlanes ? (int)(st & 1) : 0;
+      if constexpr (kPlanes) {
+        if (st + 1 < stages) {
+          stash(r, slot ^ 1);
+        }
+        if (st + 2 < stages) {
+          load_any(r, st + 2);
+        }
+      } else {
+        stash(r, 0);
+        if (st + 1 < stages) {
+          load_any(r, st + 1);
+        }
+        lds_barrier();
       }
 #pragma unroll
       for (int h = 0; h < 2; ++h) {
@@ -210,7 +227,7 @@ __global__ __launch_bounds__(kThreads, 2) void gemm_f32_mfma(
           for (int i = 0; i < 4; ++i) {
 #pragma unroll
             for (int j = 0; j < 2; ++j) {
-              if (blocks >> (2 * i + j) & 1) {
+              if (!kPlanes || (blocks >> (2 * i + j) & 1)) {
 #pragma unroll
                 for (int e = 0; e < 4; ++e) {
                   c[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(bf[j][e], af[i][e], c[i][j], 0, 0, 0);
@@ -224,202 +241,206 @@ __global__ __launch_bounds__(kThreads, 2) void gemm_f32_mfma(
     }
   };
 
-  __shared__ int again;
-  if (t == 0) {
-    again = 0;
-  }
-  /* The least magnitude but zero, as its bits times two, less one. */
-  constexpr uint32_t kTiny = 2 * kLeastBits - 1;
-  uint32_t least = ~0u;
-  auto stash = [&](const Regs &r, int slot) {
-    u32x4 p[3];
-#pragma unroll
-    for (int e = 0; e < 8; ++e) {
-      least = min(least, 2 * __float_as_uint(r.a[e]) - 1);
-      least = min(least, 2 * __float_as_uint(r.b[e]) - 1);
+  if constexpr (!kPlanes) {
+    in_f32(~0u);
+  } else {
+    __shared__ int again;
+    if (t == 0) {
+      again = 0;
     }
-    split8(r.a, p);
+    /* The least magnitude but zero, as its bits times two, less one. */
+    constexpr uint32_t kTiny = 2 * kLeastBits - 1;
+    uint32_t least = ~0u;
+    auto stash = [&](const Regs &r, int slot) {
+      u32x4 p[3];
 #pragma unroll
-    for (int i = 0; i < 3; ++i) {
-      lds[(6 * slot + i) * kPlane + unit(a_row, a_chunk)] = p[i];
-    }
-    split8(r.b, p);
-#pragma unroll
-    for (int i = 0; i < 3; ++i) {
-      lds[(6 * slot + 3 + i) * kPlane + unit(b_col, b_chunk)] = p[i];
-    }
-  };
-  f32x4 lo[4][2];
-#pragma unroll
-  for (int q = 0; q < 8; ++q) {
-    c[q >> 1][q & 1] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
-    lo[q >> 1][q & 1] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
-  }
-  u32x4 af[3][4], bf[3][2];
-  auto fragments = [&](int slot) {
-#pragma unroll
-    for (int p = 0; p < 3; ++p) {
-#pragma unroll
-      for (int j = 0; j < 2; ++j) {
-        bf[p][j] = lds[(6 * slot + 3 + p) * kPlane + unit(32 * wn + 16 * j + l16, g)];
+      for (int e = 0; e < 8; ++e) {
+        least = min(least, 2 * __float_as_uint(r.a[e]) - 1);
+        least = min(least, 2 * __float_as_uint(r.b[e]) - 1);
       }
+      split8(r.a, p);
 #pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        af[p][i] = lds[(6 * slot + p) * kPlane + unit(64 * wm + 16 * i + l16, g)];
+      for (int i = 0; i < 3; ++i) {
+        lds[(6 * slot + i) * kPlane + unit(a_row, a_chunk)] = p[i];
       }
-    }
-  };
-  auto multiply = [&]() {
-    auto add = [&](int pa_, int pb_, f32x4 (&x)[4][2]) {
+      split8(r.b, p);
 #pragma unroll
-      for (int j = 0; j < 2; ++j) {
+      for (int i = 0; i < 3; ++i) {
+        lds[(6 * slot + 3 + i) * kPlane + unit(b_col, b_chunk)] = p[i];
+      }
+    };
+    f32x4 lo[4][2];
+#pragma unroll
+    for (int q = 0; q < 8; ++q) {
+      c[q >> 1][q & 1] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+      lo[q >> 1][q & 1] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+    }
+    u32x4 af[3][4], bf[3][2];
+    auto fragments = [&](int slot) {
+#pragma unroll
+      for (int p = 0; p < 3; ++p) {
+#pragma unroll
+        for (int j = 0; j < 2; ++j) {
+          bf[p][j] = lds[(6 * slot + 3 + p) * kPlane + unit(32 * wn + 16 * j + l16, g)];
+        }
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
-          x[i][j] = mfma16<true>(bf[pb_][j], af[pa_][i], x[i][j]);
+          af[p][i] = lds[(6 * slot + p) * kPlane + unit(64 * wm + 16 * i + l16, g)];
         }
       }
     };
-    add(0, 0, c);
-    add(0, 1, lo);
-    add(1, 0, lo);
-    add(1, 1, lo);
-    add(0, 2, lo);
-    add(2, 0, lo);
-  };
+    auto multiply = [&]() {
+      auto add = [&](int pa_, int pb_, f32x4 (&x)[4][2]) {
+#pragma unroll
+        for (int j = 0; j < 2; ++j) {
+#pragma unroll
+          for (int i = 0; i < 4; ++i) {
+            x[i][j] = mfma16<true>(bf[pb_][j], af[pa_][i], x[i][j]);
+          }
+        }
+      };
+      add(0, 0, c);
+      add(0, 1, lo);
+      add(1, 0, lo);
+      add(1, 1, lo);
+      add(0, 2, lo);
+      add(2, 0, lo);
+    };
 
-  /* Entering stage s: it is in slot s % 2, the next in r[(s + 1) % 3], the one
-   * after in r[(s + 2) % 3]. */
-  Regs r[3];
-  load_any(r[0], 0);
-  if (stages > 1) {
-    load_any(r[1], 1);
-  }
-  if (stages > 2) {
-    load_any(r[2], 2);
-  }
-  stash(r[0], 0);
-  lds_barrier();
-  int64_t st = 0;
-  auto stage = [&](int64_t s, int slot, const Regs &next, Regs &after) {
-    load(after, s + 3);
-    fragments(slot);
-    multiply();
-    stash(next, slot ^ 1);
-#pragma unroll
-    for (int i = 0; i < 48; ++i) {
-      __builtin_amdgcn_sched_group_barrier(0x008, 1, 0); /* MFMA */
-      __builtin_amdgcn_sched_group_barrier(0x002, 4, 0); /* VALU */
+    /* Entering stage s: it is in slot s % 2, the next in r[(s + 1) % 3], the one
+     * after in r[(s + 2) % 3]. */
+    Regs r[3];
+    load_any(r[0], 0);
+    if (stages > 1) {
+      load_any(r[1], 1);
     }
+    if (stages > 2) {
+      load_any(r[2], 2);
+    }
+    stash(r[0], 0);
     lds_barrier();
-  };
-  for (; st + 8 < whole; st += 6) {
+    int64_t st = 0;
+    auto stage = [&](int64_t s, int slot, const Regs &next, Regs &after) {
+      load(after, s + 3);
+      fragments(slot);
+      multiply();
+      stash(next, slot ^ 1);
 #pragma unroll
-    for (int i = 0; i < 6; ++i) {
-      stage(st + i, i & 1, r[(i + 1) % 3], r[i % 3]);
+      for (int i = 0; i < 48; ++i) {
+        __builtin_amdgcn_sched_group_barrier(0x008, 1, 0); /* MFMA */
+        __builtin_amdgcn_sched_group_barrier(0x002, 4, 0); /* VALU */
+      }
+      lds_barrier();
+    };
+    for (; st + 8 < whole; st += 6) {
+#pragma unroll
+      for (int i = 0; i < 6; ++i) {
+        stage(st + i, i & 1, r[(i + 1) % 3], r[i % 3]);
+      }
     }
-  }
-  for (; st < stages; ++st) {
-    const int slot = (int)(st & 1);
-    fragments(slot);
-    if (st + 1 < stages) {
-      stash(r[1], slot ^ 1);
+    for (; st < stages; ++st) {
+      const int slot = (int)(st & 1);
+      fragments(slot);
+      if (st + 1 < stages) {
+        stash(r[1], slot ^ 1);
+      }
+      r[1] = r[2];
+      if (st + 3 < stages) {
+        load_any(r[2], st + 3);
+      }
+      multiply();
+      lds_barrier();
     }
-    r[1] = r[2];
-    if (st + 3 < stages) {
-      load_any(r[2], st + 3);
-    }
-    multiply();
-    lds_barrier();
-  }
 
-  uint32_t small = least, large = 0; /* of the sums, likewise, and the greatest */
-#pragma unroll
-  for (int q = 0; q < 8; ++q) {
-#pragma unroll
-    for (int e = 0; e < 4; ++e) {
-      const float v = c[q >> 1][q & 1][e] + lo[q >> 1][q & 1][e];
-      c[q >> 1][q & 1][e] = v;
-      small = min(small, 2 * __float_as_uint(v) - 1);
-      large = max(large, __float_as_uint(v) & 0x7fffffffu);
-    }
-  }
-  if (small < kTiny || large >= 0x7f800000u) {
-    again = 1;
-  }
-  __syncthreads();
-  if (again) {
-    /* Blocks of c to compute again (bit 2 i + j): sums that are not finite,
-     * or too small for the planes' products. */
-    uint32_t odd = 0;
+    uint32_t small = least, large = 0; /* of the sums, likewise, and the greatest */
 #pragma unroll
     for (int q = 0; q < 8; ++q) {
 #pragma unroll
       for (int e = 0; e < 4; ++e) {
-        const float v = __builtin_fabsf(c[q >> 1][q & 1][e]);
-        odd |= (uint32_t)(!(v < INFINITY) || (v > 0.0f && v < kLeast)) << q;
+        const float v = c[q >> 1][q & 1][e] + lo[q >> 1][q & 1][e];
+        c[q >> 1][q & 1][e] = v;
+        small = min(small, 2 * __float_as_uint(v) - 1);
+        large = max(large, __float_as_uint(v) & 0x7fffffffu);
       }
     }
-    if (__syncthreads_or(least < kTiny)) {
-      /* What such values may have lost, at most 2^-126 of each, against the
-       * result: the rows' and columns' greatest and least are read again. */
-      float a_max = 0.0f, b_max = 0.0f;
-      uint32_t a_min = ~0u, b_min = ~0u;
-      for (st = 0; st < stages; st += 3) {
+    if (small < kTiny || large >= 0x7f800000u) {
+      again = 1;
+    }
+    __syncthreads();
+    if (again) {
+      /* Blocks of c to compute again (bit 2 i + j): sums that are not finite,
+       * or too small for the planes' products. */
+      uint32_t odd = 0;
 #pragma unroll
-        for (int i = 0; i < 3; ++i) {
-          load_any(r[i], min(st + i, stages - 1));
-        }
-#pragma unroll
-        for (int i = 0; i < 3; ++i) {
-#pragma unroll
-          for (int e = 0; e < 8; ++e) {
-            a_max = fmaxf(a_max, __builtin_fabsf(r[i].a[e]));
-            b_max = fmaxf(b_max, __builtin_fabsf(r[i].b[e]));
-            a_min = min(a_min, 2 * __float_as_uint(r[i].a[e]) - 1);
-            b_min = min(b_min, 2 * __float_as_uint(r[i].b[e]) - 1);
-          }
-        }
-      }
-      struct Side {
-        float most, tiny; /* `tiny`: whether there is one, 1 or 0 */
-      };
-      Side *rows = reinterpret_cast<Side *>(&lds[0]); /* [4][128] each */
-      Side *cols = rows + 4 * kTile;
-      rows[a_chunk * kTile + a_row] = Side{a_max, a_min < kTiny ? 1.0f : 0.0f};
-      cols[b_chunk * kTile + b_col] = Side{b_max, b_min < kTiny ? 1.0f : 0.0f};
-      __syncthreads();
-      auto side = [&](const Side *of, int at) {
-        Side x = of[at];
-#pragma unroll
-        for (int q = 1; q < 4; ++q) {
-          x.most = fmaxf(x.most, of[q * kTile + at].most);
-          x.tiny = fmaxf(x.tiny, of[q * kTile + at].tiny);
-        }
-        return x;
-      };
-      const float lost = (float)(stages * kKs) * (kLeast * 2.0f);
-#pragma unroll
-      for (int j = 0; j < 2; ++j) {
+      for (int q = 0; q < 8; ++q) {
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
-          const Side b = side(cols, 32 * wn + 16 * j + 4 * g + e);
+          const float v = __builtin_fabsf(c[q >> 1][q & 1][e]);
+          odd |= (uint32_t)(!(v < INFINITY) || (v > 0.0f && v < kLeast)) << q;
+        }
+      }
+      if (__syncthreads_or(least < kTiny)) {
+        /* What such values may have lost, at most 2^-126 of each, against the
+         * result: the rows' and columns' greatest and least are read again. */
+        float a_max = 0.0f, b_max = 0.0f;
+        uint32_t a_min = ~0u, b_min = ~0u;
+        for (st = 0; st < stages; st += 3) {
 #pragma unroll
-          for (int i = 0; i < 4; ++i) {
-            const Side a = side(rows, 64 * wm + 16 * i + l16);
-            odd |= (uint32_t)(lost * (a.tiny * b.most + b.tiny * a.most) >
-                              __builtin_fabsf(c[i][j][e]))
-                   << (2 * i + j);
+          for (int i = 0; i < 3; ++i) {
+            load_any(r[i], min(st + i, stages - 1));
+          }
+#pragma unroll
+          for (int i = 0; i < 3; ++i) {
+#pragma unroll
+            for (int e = 0; e < 8; ++e) {
+              a_max = fmaxf(a_max, __builtin_fabsf(r[i].a[e]));
+              b_max = fmaxf(b_max, __builtin_fabsf(r[i].b[e]));
+              a_min = min(a_min, 2 * __float_as_uint(r[i].a[e]) - 1);
+              b_min = min(b_min, 2 * __float_as_uint(r[i].b[e]) - 1);
+            }
+          }
+        }
+        struct Side {
+          float most, tiny; /* `tiny`: whether there is one, 1 or 0 */
+        };
+        Side *rows = reinterpret_cast<Side *>(&lds[0]); /* [4][128] each */
+        Side *cols = rows + 4 * kTile;
+        rows[a_chunk * kTile + a_row] = Side{a_max, a_min < kTiny ? 1.0f : 0.0f};
+        cols[b_chunk * kTile + b_col] = Side{b_max, b_min < kTiny ? 1.0f : 0.0f};
+        __syncthreads();
+        auto side = [&](const Side *of, int at) {
+          Side x = of[at];
+#pragma unroll
+          for (int q = 1; q < 4; ++q) {
+            x.most = fmaxf(x.most, of[q * kTile + at].most);
+            x.tiny = fmaxf(x.tiny, of[q * kTile + at].tiny);
+          }
+          return x;
+        };
+        const float lost = (float)(stages * kKs) * (kLeast * 2.0f);
+#pragma unroll
+        for (int j = 0; j < 2; ++j) {
+#pragma unroll
+          for (int e = 0; e < 4; ++e) {
+            const Side b = side(cols, 32 * wn + 16 * j + 4 * g + e);
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+              const Side a = side(rows, 64 * wm + 16 * i + l16);
+              odd |= (uint32_t)(lost * (a.tiny * b.most + b.tiny * a.most) >
+                                __builtin_fabsf(c[i][j][e]))
+                     << (2 * i + j);
+            }
           }
         }
       }
-    }
-    uint32_t blocks = 0; /* of the wave */
+      uint32_t blocks = 0; /* of the wave */
 #pragma unroll
-    for (int q = 0; q < 8; ++q) {
-      blocks |= (uint32_t)(__builtin_amdgcn_ballot_w64((odd >> q & 1) != 0) != 0) << q;
-    }
-    if (__syncthreads_or(blocks != 0)) {
-      in_f32(blocks);
+      for (int q = 0; q < 8; ++q) {
+        blocks |= (uint32_t)(__builtin_amdgcn_ballot_w64((odd >> q & 1) != 0) != 0) << q;
+      }
+      if (__syncthreads_or(blocks != 0)) {
+        in_f32(blocks);
+      }
     }
   }
 
@@ -474,26 +495,36 @@ __global__ __launch_bounds__(kThreads, 2) void gemm_f32_mfma(
       }
     }
   }
+  /* Lanes of rows 2 r and 2 r + 1 trade a block, so that a store has whole
+   * 128-byte lines: eight rows of 32 columns. */
+  const int64_t col = n0 + 32 * wn + 16 * (l16 & 1) + 4 * g;
+  auto store = [&](int64_t row, f32x4 v) {
+    if (row < M && col < N) {
+      float *p = C + row * ldc + col;
+      if (col + 3 < N) {
+        reinterpret_cast<Four *>(p)->v = v;
+      } else {
 #pragma unroll
-  for (int i = 0; i < 4; ++i) {
-#pragma unroll
-    for (int j = 0; j < 2; ++j) {
-      const int64_t row = m0 + 64 * wm + 16 * i + l16;
-      const int64_t col = n0 + 32 * wn + 16 * j + 4 * g;
-      if (row < M && col < N) {
-        float *p = C + row * ldc + col;
-        if (col + 3 < N) {
-          reinterpret_cast<Four *>(p)->v = c[i][j];
-        } else {
-#pragma unroll
-          for (int e = 0; e < 3; ++e) {
-            if (col + e < N) {
-              p[e] = c[i][j][e];
-            }
+        for (int e = 0; e < 3; ++e) {
+          if (col + e < N) {
+            p[e] = v[e];
           }
         }
       }
     }
+  };
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    f32x4 v0, v1;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      const float other = partner<1>((l16 & 1) ? c[i][0][e] : c[i][1][e]);
+      v0[e] = (l16 & 1) ? other : c[i][0][e];
+      v1[e] = (l16 & 1) ? c[i][1][e] : other;
+    }
+    const int64_t row = m0 + 64 * wm + 16 * i + (l16 & ~1);
+    store(row, v0);
+    store(row + 1, v1);
   }
 }
 
@@ -501,7 +532,8 @@ __global__ __launch_bounds__(kThreads, 2) void gemm_f32_mfma(
 
 void gemm_f32_launch(const GemmArgs &g, int splits, char *ws, hipStream_t s) {
   const int tiles_m = (int)((g.m + kTile - 1) / kTile), tiles_n = (int)((g.n + kTile - 1) / kTile);
-  hipLaunchKernelGGL(gemm_f32_mfma, dim3((unsigned)(tiles_m * tiles_n * splits)), dim3(kThreads), 0, s,
+  const auto kernel = g.k < f32::kPlanesMinK ? gemm_f32_mfma<false> : gemm_f32_mfma<true>;
+  hipLaunchKernelGGL(kernel, dim3((unsigned)(tiles_m * tiles_n * splits)), dim3(kThreads), 0, s,
                      static_cast<const float *>(g.a), static_cast<const float *>(g.b),
                      static_cast<float *>(g.c), g.m, g.n, g.k, g.lda, g.ldb, g.ldc, tiles_m,
                      tiles_n, splits, ws);
