@@ -483,9 +483,10 @@ bool run_gemm(const vx_gemm_plan &plan, Arena *arena = nullptr, bool no_alloc = 
   g.a = a.ptr, g.b = b.ptr, g.c = c.ptr;
   g.lda = a.row_stride, g.ldb = b.row_stride, g.ldc = c.row_stride;
   g.stamp = next_stamp();
-  /* The stream-K launch keeps a workspace per stream: not for the no-alloc
-   * entry point, and not into a graph being captured. */
-  g.may_split = !no_alloc && arena == nullptr && !capturing();
+  /* The launches that divide a tile's K keep a workspace per stream: not for
+   * the no-alloc entry point, not into a graph being captured, and not under
+   * a handle of several streams. */
+  g.may_split = !no_alloc && arena == nullptr && vxk::one_stream(caller_stream) && !capturing();
 
   vxk::GemmKernel which = vxk::gemm_pick(g);
   const int forced = forced_gemm_kernel.load();

@@ -29,6 +29,11 @@
 
 namespace vxk {
 
+/* Whether a handle names one stream. hipStreamPerThread names another one in
+ * each thread, so nothing is kept by it: the launches that share a workspace
+ * along a stream would run at once. */
+inline bool one_stream(hipStream_t s) { return s != hipStreamPerThread; }
+
 /* bf16 <-> f32. bf16 is the top half of an f32; narrowing rounds to nearest
  * even, and a NaN stays a quiet NaN. */
 __host__ __device__ inline float bf16_to_f32(uint16_t h) {
