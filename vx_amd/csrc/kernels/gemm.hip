@@ -985,7 +985,7 @@ direct::Plan direct_plan(const GemmArgs &g, bool may_split, double *us) {
 
 /* The split workspace of `s`, of `bytes`, for the launches that keep tickets in
  * its first kTicketBytes; null when there is none to be had. The caller holds
- * sk_mutex, through its launch. */
+ * sk_mutex, through its launch (launches that take no workspace don't). */
 static_assert(ring::kTicketBytes == direct::kTicketBytes &&
                   f32::kTicketBytes == direct::kTicketBytes,
               "one workspace for all of them");
@@ -999,28 +999,37 @@ char *split_space(size_t bytes, hipStream_t s) {
 
 void launch_ring(const GemmArgs &g, hipStream_t s) {
   const int splits = ring::splits(g.m, g.n, g.k, device_cu_count(), g.may_split);
-  std::lock_guard<std::mutex> hold(sk_mutex);
-  char *ws = splits > 1 ? split_space((size_t)ring::ws_bytes(g.m, g.n, splits), s) : nullptr;
+  std::unique_lock<std::mutex> hold(sk_mutex, std::defer_lock);
+  char *ws = nullptr;
+  if (splits > 1) {
+    hold.lock();
+    ws = split_space((size_t)ring::ws_bytes(g.m, g.n, splits), s);
+  }
   gemm_ring_launch(g, ws ? splits : 1, ws, s);
 }
 
 void launch_f32(const GemmArgs &g, hipStream_t s) {
   const int splits = f32::splits(g.m, g.n, g.k, device_cu_count(), g.may_split);
-  std::lock_guard<std::mutex> hold(sk_mutex);
-  char *ws = splits > 1 ? split_space((size_t)(f32::kTicketBytes + f32::tiles(g.m, g.n) * splits *
-                                                                       (int64_t)f32::kPart),
-                                      s)
-                        : nullptr;
+  std::unique_lock<std::mutex> hold(sk_mutex, std::defer_lock);
+  char *ws = nullptr;
+  if (splits > 1) {
+    hold.lock();
+    ws = split_space((size_t)f32::ws_bytes(g.m, g.n, splits), s);
+  }
   gemm_f32_launch(g, ws ? splits : 1, ws, s);
 }
 
 void launch_direct(const GemmArgs &g, hipStream_t s) {
   double us;
   direct::Plan plan = direct_plan(g, g.may_split, &us);
-  std::lock_guard<std::mutex> hold(sk_mutex);
-  char *ws = plan.ws_bytes ? split_space((size_t)plan.ws_bytes, s) : nullptr;
-  if (plan.ws_bytes && !ws) {
-    plan = direct_plan(g, false, &us);
+  std::unique_lock<std::mutex> hold(sk_mutex, std::defer_lock);
+  char *ws = nullptr;
+  if (plan.ws_bytes) {
+    hold.lock();
+    ws = split_space((size_t)plan.ws_bytes, s);
+    if (!ws) {
+      plan = direct_plan(g, false, &us);
+    }
   }
   gemm_direct_launch(g, plan, ws, s);
 }

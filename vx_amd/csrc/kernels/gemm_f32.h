@@ -25,6 +25,9 @@ constexpr int64_t kPlanesMinK = 128;
 inline int64_t tiles(int64_t m, int64_t n) {
   return ((m + kTile - 1) / kTile) * ((n + kTile - 1) / kTile);
 }
+inline int64_t ws_bytes(int64_t m, int64_t n, int splits) {
+  return kTicketBytes + tiles(m, n) * splits * (int64_t)kPart;
+}
 
 /* Splits of least time on a 256-CU MI355X (one workgroup to a CU): 1.15 us a
  * stage of K, 4 a round, and for a split its sums' way to memory and back. */
