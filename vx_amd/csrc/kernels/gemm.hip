@@ -47,9 +47,11 @@
 
 namespace vxk {
 
-/* gemm_direct.hip */
+/* gemm_direct.hip, gemm_ring.hip, gemm_f32.hip; `ws`: gemm_split.h */
 bool gemm_direct_takes(const GemmArgs &g);
 void gemm_direct_launch(const GemmArgs &g, const direct::Plan &plan, char *ws, hipStream_t s);
+void gemm_ring_launch(const GemmArgs &g, int splits, char *ws, hipStream_t s);
+void gemm_f32_launch(const GemmArgs &g, int splits, char *ws, hipStream_t s);
 
 namespace {
 
@@ -984,16 +986,13 @@ direct::Plan direct_plan(const GemmArgs &g, bool may_split, double *us) {
 }
 
 /* The split workspace of `s`, of `bytes`, for the launches that keep tickets in
- * its first kTicketBytes; null when there is none to be had. The caller holds
+ * its first split::kTicketBytes; null when there is none to be had. The caller holds
  * sk_mutex, through its launch (launches that take no workspace don't). */
-static_assert(ring::kTicketBytes == direct::kTicketBytes &&
-                  f32::kTicketBytes == direct::kTicketBytes,
-              "one workspace for all of them");
 char *split_space(size_t bytes, hipStream_t s) {
   int dev = 0;
   VX_HIP_CHECK(hipGetDevice(&dev));
   SkSpace &sp = sk_spaces()[{dev, s}];
-  return sk_reserve(sp.split, sp.split_bytes, bytes, (size_t)direct::kTicketBytes, s) ? sp.split
+  return sk_reserve(sp.split, sp.split_bytes, bytes, (size_t)split::kTicketBytes, s) ? sp.split
                                                                                        : nullptr;
 }
 

@@ -5,16 +5,13 @@
 #ifndef VX_AMD_GEMM_DIRECT_H
 #define VX_AMD_GEMM_DIRECT_H
 
+#include "gemm_split.h"
+
 #include <algorithm>
 #include <cstdint>
 
 namespace vxk {
 namespace direct {
-
-/* A split launch's workspace: a ticket per tile, zero between launches, then
- * the partial sums. */
-constexpr int kMaxSplitTiles = 1024;
-constexpr int64_t kTicketBytes = kMaxSplitTiles * 4;
 
 struct Plan {
   int mt;           /* 16-row blocks per wave: 1, 2 or 4 */
@@ -70,7 +67,7 @@ inline Plan plan(int64_t m, int64_t n, int64_t k, bool odd, int cus, bool may_sp
       best.tiles_m = (int)tiles_m;
       best.tiles_n = tiles_n;
       best.splits = (int)splits;
-      best.ws_bytes = splits > 1 ? kTicketBytes + tiles * splits * (int64_t)(mt * 16 * 128 * 4) : 0;
+      best.ws_bytes = splits > 1 ? split::kTicketBytes + tiles * splits * (int64_t)(mt * 16 * 128 * 4) : 0;
     }
   };
   consider(4, false, 256, 1);
@@ -82,7 +79,7 @@ inline Plan plan(int64_t m, int64_t n, int64_t k, bool odd, int cus, bool may_sp
     const int64_t tiles = (m + 16 * mt - 1) / (16 * mt) * tiles_n;
     /* one workgroup per CU, of at least 4 blocks of k a wave */
     const int64_t splits = std::min<int64_t>(cus / tiles, k / 512);
-    if (may_split && splits > 1 && tiles <= kMaxSplitTiles) {
+    if (may_split && splits > 1 && tiles <= split::kMaxTiles) {
       consider(mt, true, 16 * mt, splits);
     }
   }

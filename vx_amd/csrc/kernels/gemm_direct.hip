@@ -314,7 +314,7 @@ __global__ __launch_bounds__(kThreads, kMT <= 2 ? 2 : 1) void gemm_direct(Direct
      * before the ticket. */
     constexpr int kPart = 8 * kMT * 64 * 16; /* bytes of one split's sums of a tile */
     const __amdgpu_buffer_rsrc_t wr = __builtin_amdgcn_make_buffer_rsrc(
-        (void *)(p.ws + direct::kTicketBytes + (int64_t)tile * p.splits * kPart), (short)0,
+        (void *)(p.ws + split::kTicketBytes + (int64_t)tile * p.splits * kPart), (short)0,
         p.splits * kPart, 0x00020000);
     const int at = (wave * 2 * kMT * 64 + lane) * 16;
 #pragma unroll

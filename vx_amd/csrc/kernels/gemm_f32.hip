@@ -448,7 +448,7 @@ __global__ __launch_bounds__(kThreads, kPlanes ? 2 : 6) void gemm_f32_mfma(
     /* The sums go past the caches that other XCDs do not see; the workgroup
      * with the last ticket adds all of them up in order. */
     const __amdgpu_buffer_rsrc_t wr = __builtin_amdgcn_make_buffer_rsrc(
-        (void *)(ws + f32::kTicketBytes + (int64_t)id * splits * f32::kPart), (short)0,
+        (void *)(ws + split::kTicketBytes + (int64_t)id * splits * f32::kPart), (short)0,
         splits * f32::kPart, 0x00020000);
     const int at = t * 16;
     __shared__ int last;

@@ -1,11 +1,11 @@
 /*
- * gemm_ring.h -- launcher of the 128x128- and 256x128-tile GEMM (gemm_ring.hip)
- * and the choice of its tile and splits. Plain host arithmetic.
+ * gemm_ring.h -- the choice of tile and splits of the 128x128- and 256x128-tile
+ * GEMM (gemm_ring.hip). Plain host arithmetic.
  */
 #ifndef VX_AMD_GEMM_RING_H
 #define VX_AMD_GEMM_RING_H
 
-#include "../vx_kernels.h"
+#include "gemm_split.h"
 
 #include <algorithm>
 
@@ -13,16 +13,12 @@ namespace vxk {
 namespace ring {
 
 constexpr int kTile = 128;
-/* A split launch's workspace: a ticket per tile, zero between launches, then
- * the partial sums. */
-constexpr int kMaxSplitTiles = 1024;
-constexpr int64_t kTicketBytes = kMaxSplitTiles * 4;
 
 inline int64_t tiles(int64_t m, int64_t n) {
   return ((m + kTile - 1) / kTile) * ((n + kTile - 1) / kTile);
 }
 inline int64_t ws_bytes(int64_t m, int64_t n, int splits) {
-  return kTicketBytes + tiles(m, n) * splits * (int64_t)(kTile * kTile * 4);
+  return split::kTicketBytes + tiles(m, n) * splits * (int64_t)(kTile * kTile * 4);
 }
 
 /* Microseconds on a 256-CU MI355X: a stage of K takes 0.53 where CUs have two
@@ -55,8 +51,8 @@ inline bool tall(int64_t m, int64_t n, int64_t k, int cus) {
 /* Splits of least time by that model. */
 inline int splits(int64_t m, int64_t n, int64_t k, int cus, bool may_split) {
   int best = 1;
-  if (may_split && tiles(m, n) <= kMaxSplitTiles) {
-    for (int s = 2; s <= 8 && k / 32 / s >= 8; ++s) {
+  if (may_split && tiles(m, n) <= split::kMaxTiles) {
+    for (int s = 2; s <= 8 && k / 32 / s >= 8 && ws_bytes(m, n, s) <= split::kMaxBytes; ++s) {
       if (us(m, n, k, s, cus) < us(m, n, k, best, cus)) {
         best = s;
       }
@@ -66,8 +62,6 @@ inline int splits(int64_t m, int64_t n, int64_t k, int cus, bool may_split) {
 }
 
 } // namespace ring
-
-void gemm_ring_launch(const GemmArgs &g, int splits, char *ws, hipStream_t s);
 
 } // namespace vxk
 

@@ -215,7 +215,7 @@ __global__ __launch_bounds__(2 * kBM, 2) void gemm_ring(
 
   if (kBM == ring::kTile && splits > 1) {
     const __amdgpu_buffer_rsrc_t wr = __builtin_amdgcn_make_buffer_rsrc(
-        (void *)(ws + ring::kTicketBytes + (int64_t)id * splits * kPart), (short)0,
+        (void *)(ws + split::kTicketBytes + (int64_t)id * splits * kPart), (short)0,
         splits * kPart, 0x00020000);
     /* in the ring, whose reads are done after the barrier: with a word more
      * LDS than 80 KiB a CU has room for one workgroup only */
