@@ -360,8 +360,9 @@ std::atomic<int64_t> stat_image_launches{0};
 std::atomic<int64_t> stat_image_loads{0};
 std::atomic<int> forced_gemm_kernel{0};
 
-/* Clock stamps of routed MFMA GEMMs (VX_HIP_CTRL_CLOCK_STAMPS): a ring of
- * `slots` records of 4 u64 in HBM, one per launch in turn; off when null. */
+/* Clock stamps of routed 16-bit MFMA GEMMs (VX_HIP_CTRL_CLOCK_STAMPS): a ring of
+ * `slots` records of 4 u64 in HBM, one per launch in turn (other launches leave
+ * theirs as it was); off when null. */
 std::mutex stamps_mutex;
 uint64_t *stamps_base = nullptr;
 int64_t stamps_slots = 0, stamps_next = 0;

@@ -29,6 +29,7 @@
 #include "../vx_hip_common.h"
 #include "../vx_kernels.h"
 #include "gemm_direct.h"
+#include "vx_clock_stamp.hip.h"
 #include "vx_mfma16.hip.h"
 
 #include <algorithm>
@@ -56,6 +57,7 @@ struct DirectArgs {
   int tiles_m, tiles_n;
   int splits;
   char *ws;
+  uint64_t *stamp;
 };
 
 /* Eight consecutive columns of a row of C. */
@@ -82,6 +84,7 @@ template <int kOut> __device__ __forceinline__ void put8(char *c, int64_t at, co
 
 template <bool kBf16, int kOut, int kMT, int kBuf, bool kAlongK, bool kOddA>
 __global__ __launch_bounds__(kThreads, kMT <= 2 ? 2 : 1) void gemm_direct(DirectArgs p) {
+  const ClockStamp clocks(p.stamp);
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int l16 = lane & 15;
@@ -283,6 +286,7 @@ __global__ __launch_bounds__(kThreads, kMT <= 2 ? 2 : 1) void gemm_direct(Direct
         store(t, r, v);
       }
     }
+    clocks.end();
     return;
   }
 
@@ -335,6 +339,7 @@ __global__ __launch_bounds__(kThreads, kMT <= 2 ? 2 : 1) void gemm_direct(Direct
     }
     __syncthreads();
     if (!last) {
+      clocks.end();
       return;
     }
     f32x4 sum[2 * kMT];
@@ -370,6 +375,7 @@ __global__ __launch_bounds__(kThreads, kMT <= 2 ? 2 : 1) void gemm_direct(Direct
     }
     store(tr >> 2, tr & 3, v);
   }
+  clocks.end();
 }
 
 /* kBuf blocks of a wave's loads in flight, as its registers allow: kBufOdd for
@@ -422,6 +428,7 @@ void gemm_direct_launch(const GemmArgs &g, const direct::Plan &plan, char *ws, h
   p.m = g.m, p.n = g.n, p.k = (int)g.k;
   p.tiles_m = plan.tiles_m, p.tiles_n = plan.tiles_n, p.splits = plan.splits;
   p.ws = ws;
+  p.stamp = g.stamp;
   const bool bf = g.in_dtype == VX_DTYPE_BF16;
   if (g.out_dtype == VX_DTYPE_F32) {
     bf ? launch_plan<true, VX_DTYPE_F32>(p, plan, s) : launch_plan<false, VX_DTYPE_F32>(p, plan, s);

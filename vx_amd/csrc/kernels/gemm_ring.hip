@@ -26,6 +26,7 @@
 #include "../vx_kernels.h"
 #include "gemm_pp_layout.h"
 #include "gemm_ring.h"
+#include "vx_clock_stamp.hip.h"
 #include "vx_lds_dma.hip.h"
 #include "vx_mfma16.hip.h"
 
@@ -73,7 +74,8 @@ template <bool kBf16, int kOut, int kBM>
 __global__ __launch_bounds__(2 * kBM, 2) void gemm_ring(
     const uint16_t *__restrict__ A, const uint16_t *__restrict__ B, void *__restrict__ C,
     int64_t M, int64_t N, int K, int64_t lda, int64_t ldb, int64_t ldc, int tiles_m,
-    int tiles_n, int splits, char *__restrict__ ws) {
+    int tiles_n, int splits, char *__restrict__ ws, uint64_t *__restrict__ stamp) {
+  const ClockStamp clocks(stamp);
   constexpr int kThreads = 2 * kBM;                         /* a wave per 64x64 */
   constexpr int kNS = kBM == 128 ? 5 : 6;                   /* slots: 80 KiB, or 144 */
   constexpr int kUA = kBM * 4;                              /* 16-byte units per stage */
@@ -242,6 +244,7 @@ __global__ __launch_bounds__(2 * kBM, 2) void gemm_ring(
     }
     __syncthreads();
     if (!last) {
+      clocks.end();
       return;
     }
     for (int s2 = 0; s2 < splits; ++s2) {
@@ -277,6 +280,7 @@ __global__ __launch_bounds__(2 * kBM, 2) void gemm_ring(
       }
     }
   }
+  clocks.end();
 }
 
 template <bool kBf16, int kOut, int kBM>
@@ -284,7 +288,8 @@ void launch_rows(const GemmArgs &g, int splits, char *ws, hipStream_t s) {
   const int tiles_m = (int)((g.m + kBM - 1) / kBM), tiles_n = (int)((g.n + kBN - 1) / kBN);
   hipLaunchKernelGGL((gemm_ring<kBf16, kOut, kBM>), dim3(tiles_m * tiles_n * splits),
                      dim3(2 * kBM), 0, s, static_cast<const uint16_t *>(g.a), static_cast<const uint16_t *>(g.b),
-                     g.c, g.m, g.n, (int)g.k, g.lda, g.ldb, g.ldc, tiles_m, tiles_n, splits, ws);
+                     g.c, g.m, g.n, (int)g.k, g.lda, g.ldb, g.ldc, tiles_m, tiles_n, splits, ws,
+                     g.stamp);
 }
 
 template <bool kBf16, int kOut>

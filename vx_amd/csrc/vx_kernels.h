@@ -25,7 +25,7 @@ struct GemmArgs {
   const void *b;
   void *c;
   int64_t lda, ldb, ldc;
-  /* Where the MFMA kernel records its clock counters (4 x u64: shader clock
+  /* Where a 16-bit MFMA kernel records its clock counters (4 x u64: shader clock
    * and real-time counter at the start and end of workgroup 0), or null. */
   uint64_t *stamp = nullptr;
   /* Whether the launch may take a workspace of its own (false under graph

@@ -160,7 +160,7 @@ class DispatchLibrary:
             raise ValueError(f"no flash-attention split count {splits}")
 
     def clock_stamps(self, base: int | None, slots: int) -> None:
-        """Have routed MFMA GEMMs record their clock counters (4 x u64 per
+        """Have routed 16-bit MFMA GEMMs record their clock counters (4 x u64 per
         launch: shader clock and 100 MHz real-time counter at the start and
         end of workgroup 0) into a ring of `slots` records at the HBM address
         `base`; base None stops it."""
