@@ -1,5 +1,6 @@
 """The attention launch whose workgroups' halves divide the keys
-(flash_attn.hip, two groups), at the edges of its blocks, against the oracle."""
+(flash_attn.hip, two groups), at the edges of its blocks, and the undivided
+one of one group, against the oracle."""
 
 import numpy as np
 import pytest
@@ -7,7 +8,7 @@ import pytest
 import oracle
 from tests.conftest import announce
 from tests.parity import BF16_ABS, assert_max_abs
-from tests.test_gpu_flash_attn import randn16, run
+from tests.test_gpu_flash_attn import CASES, randn16, run
 
 pytestmark = pytest.mark.gpu
 
@@ -15,12 +16,17 @@ pytestmark = pytest.mark.gpu
 @pytest.mark.parametrize("causal", [True, False])
 @pytest.mark.parametrize("case", [
     # batch, heads, kv_heads, seq_q, seq_k, head_dim; 64-key blocks
-    (1, 2, 1, 33, 64, 64),     # one block: the second half sees none
-    (1, 3, 3, 64, 65, 128),    # a second block of one key
+    (1, 2, 1, 33, 64, 64),     # one block: one group
+    (1, 3, 3, 64, 65, 128),    # two blocks of head size 128: one group
+    (1, 2, 1, 33, 65, 64),     # a second block of one key
+    (1, 3, 3, 64, 193, 128),   # a fourth block of one key
+    (2, 3, 1, 100, 100, 64),   # causal: the first queries' second half sees none
+    (1, 2, 2, 300, 200, 128),  # more queries than keys, four blocks
+    (1, 200, 50, 129, 320, 64),  # more than half a round: five blocks
     (2, 4, 2, 65, 129, 64),    # three blocks, a second workgroup of one query
     (1, 2, 2, 200, 256, 128),  # four blocks
     (1, 2, 2, 300, 70, 64),    # more queries than keys: rows that see none
-    (1, 2, 2, 300, 70, 128),
+    (1, 2, 2, 300, 70, 128),   # one group
     (1, 4, 1, 700, 1000, 64),  # many blocks, a tail of 40 keys
     (1, 16, 4, 260, 260, 128)])
 def test_two_groups_match_oracle(hiplib, case, causal, rng):
@@ -36,3 +42,26 @@ def test_two_groups_match_oracle(hiplib, case, causal, rng):
         assert np.array_equal(np.isfinite(lse.ravel()), seen)
         assert_max_abs(lse.ravel()[seen], wl[seen], 1e-3, f"lse {case}")
         assert np.all(o.reshape(-1, d)[~seen] == 0)
+
+
+@pytest.mark.parametrize("causal", [True, False])
+@pytest.mark.parametrize("case", CASES + [
+    (1, 2, 1, 33, 64, 64), (1, 3, 3, 64, 65, 64), (1, 2, 2, 300, 70, 64), (1, 4, 1, 700, 1000, 64),
+    (1, 4, 1, 300, 457, 128), (2, 4, 2, 129, 513, 64)])
+def test_one_group_matches_oracle(hiplib, case, causal, rng):
+    """The undivided launch of 128-query workgroups, which larger grids take:
+    a forced split count of 1."""
+    announce(f"flash attn one group {case} causal={causal}")
+    b, h, hk, sq, sk, d = case
+    q16, k16, v16 = randn16(rng, (b, h, sq, d)), randn16(rng, (b, hk, sk, d)), randn16(rng, (b, hk, sk, d))
+    hiplib.force_fa_splits(1)
+    try:
+        o, lse = run(hiplib, q16, k16, v16, h, hk, d ** -0.5, causal, poison=True)
+    finally:
+        hiplib.force_fa_splits(0)
+    wo, wl = oracle.attention_rows(q16, k16, v16, h, hk, d ** -0.5, causal, oracle.attention_all_rows(b, h, sq))
+    assert_max_abs(o.reshape(-1, d), wo, BF16_ABS, f"o {case}")
+    seen = np.isfinite(wl)
+    assert np.array_equal(np.isfinite(lse.ravel()), seen)
+    assert_max_abs(lse.ravel()[seen], wl[seen], 1e-3, f"lse {case}")
+    assert np.all(o.reshape(-1, d)[~seen] == 0)

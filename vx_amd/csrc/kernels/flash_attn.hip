@@ -814,13 +814,14 @@ int pick_splits(int64_t items, int64_t key_blocks, int cus) {
  * against 61). Head size 128 (one to a CU): up to one round, where the keys
  * would not be cut (8 heads, 1000^2 24.2 -> 19.0; 512 queries of 32 heads over
  * 512 keys 15.9 -> 13.5, over 2048 in 2 splits 36.0 against 35.1, over 8192 in
- * 4 splits 87 against 125). */
+ * 4 splits 87 against 125). Undivided launches (`allow_split` false) are not
+ * cut, and a forced number of splits has no groups. */
 bool two_groups(int head_dim, int64_t items, int64_t items64, int64_t key_blocks, int cus,
                 bool allow_split) {
-  if (allow_split && forced_splits.load() > 1) {
+  if (forced_splits.load() > 0) {
     return false;
   }
-  const int splits = auto_splits(items, key_blocks, cus);
+  const int splits = allow_split ? auto_splits(items, key_blocks, cus) : 1;
   return head_dim == 64 ? items64 <= 2 * cus && splits < 4 : items64 <= cus && splits == 1;
 }
 

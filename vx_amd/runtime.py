@@ -154,7 +154,7 @@ class DispatchLibrary:
 
     def force_fa_splits(self, splits: int) -> None:
         """Cut every flash-attention launch's key range into `splits` parts
-        (0: the automatic choice; graph capture always runs unsplit)."""
+        (0: the automatic choice; 1, and graph capture with any, runs undivided)."""
         v = ctypes.c_int32(splits)
         if not self.lib.vx_plugin_control(abi.HIP_CTRL_FA_SPLITS, ctypes.byref(v)):
             raise ValueError(f"no flash-attention split count {splits}")
