@@ -65,3 +65,25 @@ def test_one_group_matches_oracle(hiplib, case, causal, rng):
     assert np.array_equal(np.isfinite(lse.ravel()), seen)
     assert_max_abs(lse.ravel()[seen], wl[seen], 1e-3, f"lse {case}")
     assert np.all(o.reshape(-1, d)[~seen] == 0)
+
+
+@pytest.mark.parametrize("causal", [True, False])
+@pytest.mark.parametrize("case", [
+    # batch, heads, kv_heads, seq_q, seq_k, head_dim: each side of the choice
+    (1, 64, 32, 513, 577, 64), (1, 64, 8, 512, 577, 64),  # past one round of two groups, and one
+    (2, 32, 8, 300, 300, 128), (1, 32, 8, 500, 512, 128),
+    (64, 32, 32, 20, 130, 128), (16, 32, 4, 9, 130, 128),  # one group, few rows
+    (4, 128, 32, 20, 255, 64), (4, 129, 43, 20, 255, 64),
+    (1, 256, 256, 17, 384, 128), (1, 255, 255, 17, 384, 128)])
+def test_grids_beside_the_choices(hiplib, case, causal, rng):
+    announce(f"flash attn grids {case} causal={causal}")
+    b, h, hk, sq, sk, d = case
+    q16, k16, v16 = randn16(rng, (b, h, sq, d)), randn16(rng, (b, hk, sk, d)), randn16(rng, (b, hk, sk, d))
+    o, lse = run(hiplib, q16, k16, v16, h, hk, d ** -0.5, causal, poison=True)
+    assert np.isfinite(o).all() and np.isfinite(lse).all()
+    rows = np.array(sorted({(bi, hi, qi) for bi in (0, b - 1) for hi in range(0, h, max(1, h // 16))
+                            for qi in {0, sq - 1, *rng.integers(0, sq, 6).tolist()}}), np.int64)
+    wo, wl = oracle.attention_rows(q16, k16, v16, h, hk, d ** -0.5, causal, rows)
+    at = (rows[:, 0], rows[:, 1], rows[:, 2])
+    assert_max_abs(o[at], wo, BF16_ABS, f"o {case}")
+    assert_max_abs(lse[at], wl, 1e-3, f"lse {case}")

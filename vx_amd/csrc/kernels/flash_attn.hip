@@ -806,23 +806,35 @@ int pick_splits(int64_t items, int64_t key_blocks, int cus) {
 
 /* Whether workgroups of 64 queries, whose two halves divide the keys, take the
  * call: `items` 128-query and `items64` 64-query workgroups. They give a small
- * grid twice the workgroups without partial results in memory, and load each
- * key twice as often. Head size 64 (two to a CU): up to one round, where the
- * keys would be cut less than four ways (16 heads, 2048^2 causal 33.3 -> 21.8
- * us, 8 heads, 1000^2 18.0 -> 12.0; 1024 workgroups, 2 x 32 heads, 1024^2 30.1
- * against 33.5; 128 queries of 32 heads over 8000 keys in 8 splits 28.1
- * against 61). Head size 128 (one to a CU): up to one round, where the keys
- * would not be cut (8 heads, 1000^2 24.2 -> 19.0; 512 queries of 32 heads over
- * 512 keys 15.9 -> 13.5, over 2048 in 2 splits 36.0 against 35.1, over 8192 in
- * 4 splits 87 against 125). Undivided launches (`allow_split` false) are not
- * cut, and a forced number of splits has no groups. */
-bool two_groups(int head_dim, int64_t items, int64_t items64, int64_t key_blocks, int cus,
-                bool allow_split) {
+ * grid twice the workgroups without partial results in memory, load each key
+ * twice as often, and pay for where the halves meet; a forced number of splits
+ * has none of them. One group and two, causal, us:
+ * Head size 64 (two to a CU): up to one round, of more blocks of keys where it
+ * is more than half full and waves have their 32 queries (8 heads, 1000 queries
+ * over 128 keys 5.8 -> 5.2, 64 heads, 512 queries 6.1 against 6.9, 300 queries
+ * over 512 keys 11.2 -> 10.0; 512 heads, 16 queries over 100 6.3 -> 5.7),
+ * where the keys would not be cut three ways or more (4 heads, 64 queries over
+ * 4000 keys in 3 splits 23.7 against 32.5; 256 workgroups 37.4 -> 35.5).
+ * Head size 128 (one to a CU): up to one round, and half of one where they are
+ * not more than one group's and the keys few (64 queries a head over 512 keys,
+ * 128 heads 14.8 -> 13.8, 256 heads 17.1 against 17.4, 33 over 1500 36.8 ->
+ * 33.2), from 4 blocks of keys on (8 heads, 200 queries over 100 keys 6.9
+ * against 7.6, 1000 over 256 9.9 -> 9.1), where the keys would not be cut (512
+ * queries of 32 heads over 2048 keys in 2 splits 36.0 against 35.1, over 8192
+ * in 4 splits 87 against 125). Undivided launches (`allow_split` false) are
+ * not cut. */
+bool two_groups(int head_dim, int64_t seq_q, int64_t items, int64_t items64, int64_t key_blocks,
+                int cus, bool allow_split) {
   if (forced_splits.load() > 0) {
     return false;
   }
   const int splits = allow_split ? auto_splits(items, key_blocks, cus) : 1;
-  return head_dim == 64 ? items64 <= 2 * cus && splits < 4 : items64 <= cus && splits == 1;
+  if (head_dim == 64) {
+    return items64 <= 2 * cus && key_blocks >= (items64 <= cus || seq_q <= 32 ? 2 : 5) &&
+           (splits < 3 || (splits == 3 && items64 > cus / 2));
+  }
+  return items64 <= (items64 > items || key_blocks >= 16 ? cus : cus / 2) && key_blocks >= 4 &&
+         splits == 1;
 }
 
 /* Split partials of one (device, stream). Launches on one stream run in
@@ -1002,8 +1014,8 @@ bool flash_attn_fwd_launch(const uint16_t *q, const uint16_t *k,
   if (items * splits > INT32_MAX || bh * seq_q * (head_dim / 4) > INT32_MAX) {
     splits = 1;
   }
-  if (two_groups((int)head_dim, items, bh * ((seq_q + 63) / 64), key_blocks, device_cu_count(),
-                 allow_split)) {
+  if (two_groups((int)head_dim, seq_q, items, bh * ((seq_q + 63) / 64), key_blocks,
+                 device_cu_count(), allow_split)) {
     splits = 0;
   }
   if (splits > 1) {
