@@ -877,14 +877,36 @@ bool reserve(char *&base, size_t &held, size_t bytes, size_t zeroed, hipStream_t
   return true;
 }
 
-/* Calls of up to kRowsMaxQ queries a head over at least kRowsMinK keys: all of
- * a KV head's heads together (flash_rows.hip), where this kernel would give
- * each head a workgroup of 128 rows. With 16 x 64 heads on 8, d 128, over 4096
- * keys: 16 queries 308 -> 105 us, 32 queries 312 -> 208 (at 64 this kernel's
- * rate, twice that of 32, is the higher). Over 31 keys its one launch of 24
- * workgroups takes 5.5 us and flash_rows 6.3. */
+/* Whether flash_rows.hip takes a call: up to kRowsMaxQ queries a head over at
+ * least kRowsMinK keys, all of a KV head's heads together, where this kernel
+ * would give each of `heads` in all a workgroup of 128 rows. With 16 x 64 heads
+ * on 8, d 128, over 4096 keys: 16 queries 308 -> 105 us, 32 queries 312 -> 208
+ * (at 64 this kernel's rate, twice that of 32, is the higher). Over 31 keys its
+ * one launch of 24 workgroups takes 5.5 us and flash_rows 6.3.
+ * Its tiles of 32 rows (more than 16 of a KV head) start slower, which few keys
+ * do not make up for (32 heads, 32 queries, d 128: 128 keys 6.0 us against 6.9;
+ * 16 heads over 512 keys 12.3 -> 11.1) unless the heads' own workgroups would
+ * take a round of two to a CU (of 16 queries; of up to 32 at head size 64: 8
+ * heads on each of 128, 20 queries over 190 keys 16.1 -> 11.7). A head of its
+ * own on each KV head and a full grid: this kernel reads K and V once as well
+ * (256 x 32 heads, 32 queries over 128 keys 140 against 222; 512 heads, 20 over
+ * 1024 44 against 47; 16 x 32 heads, 32 over 2048 101 -> 96). */
 constexpr int kRowsMaxQ = 32;
 constexpr int kRowsMinK = 128;
+
+bool rows_take(int head_dim, int64_t heads, int64_t kv_total, int64_t rows, int64_t seq_q,
+               int64_t seq_k, int cus) {
+  if (seq_q > kRowsMaxQ || seq_k < kRowsMinK) {
+    return false;
+  }
+  if (rows <= 16) {
+    return true;
+  }
+  if (seq_k < (head_dim == 64 ? 256 : 384)) {
+    return seq_q <= 16 ? heads >= 2 * cus : head_dim == 64 && heads > 2 * cus;
+  }
+  return !(head_dim == 128 && heads == kv_total && heads >= cus && seq_k < 2048);
+}
 
 rows::Plan rows_plan(int64_t kv_total, int64_t rows, int64_t seq_k, int head_dim, int cus,
                      bool allow_split) {
@@ -981,7 +1003,8 @@ bool flash_attn_fwd_launch(const uint16_t *q, const uint16_t *k,
   }
   const float scale_log2 = scale * 1.4426950408889634f;
   const int group = (int)(heads / kv_heads);
-  if (seq_q <= kRowsMaxQ && seq_k >= kRowsMinK) {
+  if (rows_take((int)head_dim, bh, batch * kv_heads, group * seq_q, seq_q, seq_k,
+                device_cu_count())) {
     rows::Args a{q, k, v, o, lse, batch * kv_heads, group * (int)seq_q, (int)seq_q, (int)seq_k,
                  scale_log2, causal};
     rows::Plan plan = rows_plan(a.kv_total, a.rows, seq_k, (int)head_dim, device_cu_count(),
