@@ -44,7 +44,17 @@ static void check(int64_t m, int64_t n, int64_t k) {
   }
 }
 
+// Few k over many rounds: 64-row tiles, one to a CU, take twice the time.
+static void check_short(int64_t m, int64_t n, int64_t k) {
+  double us;
+  const vxk::direct::Plan d = vxk::direct::plan(m, n, k, k % 2 != 0, 256, true, &us);
+  expect(!(d.along_k && d.mt == 4), "64-row tiles", m, n, k);
+}
+
 int main() {
+  check_short(146800, 40, 16);
+  check_short(15296, 832, 9);
+  check_short(1390, 41136, 5);
   check(2176, 7552, 262144);
   check(1920, 8192, 262144);
   check(128 * 1024, 128, 1 << 20); // as many tiles as tickets

@@ -30,10 +30,10 @@ inline bool shape_ok(int64_t m, int64_t n, int64_t k, int64_t lda, int64_t ldb, 
 }
 
 /* Microseconds, from times on a 256-CU MI355X (4 to 8192 rows, K 64 to 12000,
- * within a third of the measured): a launch takes 3, and a wave one block of
- * 32 k in `block`; an A off the 4-byte grid is loaded in words. Two operands
- * of 4000^3, for instance: 128 blocks on two rounds of 256-row tiles 215,
- * with odd rows 340. */
+ * within a third of the measured; 8 to 400000 rows and columns, K 1 to 127): a
+ * launch takes 3, and a wave one block of 32 k in `block`; an A off the 4-byte
+ * grid is loaded in words. Two operands of 4000^3, for instance: 128 blocks on
+ * two rounds of 256-row tiles 215, with odd rows 340. */
 inline double block_us(int mt, bool along_k, bool odd) {
   if (!along_k) {
     return odd ? 1.3 : 0.77;
@@ -57,6 +57,12 @@ inline Plan plan(int64_t m, int64_t n, int64_t k, bool odd, int cus, bool may_sp
     const int64_t rounds = (tiles * splits + cus - 1) / cus;
     double t = 3.0 + (double)rounds * (along_k ? 0.5 + 0.5 * mt + blocks / (double)(4 * splits) * block_us(mt, true, odd)
                                                : 9.0 + blocks * block_us(mt, false, odd));
+    if (along_k && mt == 4) {
+      /* one to a CU: nothing covers a round's start and store (146800 x 40 x 16
+       * in 9 rounds of these 46.8, in 3 of 256 rows 19.2); on two rounds the
+       * time above is close (124 x 22574 x 648 27.4, in 32-row tiles 33.5) */
+      t += 2.0 * (double)std::max<int64_t>(rounds - 2, 0);
+    }
     if (splits > 1) {
       t += 1.0 + 0.6 * mt + 0.05 * (double)(splits * mt); /* the ticket, the other splits' sums */
     }
