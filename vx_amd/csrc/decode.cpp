@@ -35,7 +35,11 @@ constexpr int kGraphSteps = VX_DEC_GRAPH_STEPS;
 /* Given positions from which they go together (prefill) rather than step by
  * step, in a prompt and in a scored text: at the dim-768, 12-layer decoder 2,
  * 3 and 4 prompt tokens and one new one take 418, 624 and 803 us in steps and
- * 525 together; the logits of 1, 2 and 3 tokens 295, 541 and 802, and 525. */
+ * 525 together; the logits of 1, 2 and 3 tokens 295, 541 and 802, and 525. The
+ * lines lie there at other widths and depths too (3 prompt tokens, 2 scored, in
+ * steps and together): dim 64, 2 layers 165 and 114, 149 and 63; 288, 6 layers
+ * 318 and 233, 324 and 210; 2048, 4 layers 374 and 333, 328 and 322; 4096, 2
+ * layers 416 and 291, 326 and 273. */
 constexpr int kPrefillMin = 3;
 constexpr int kScoreMin = 2;
 
