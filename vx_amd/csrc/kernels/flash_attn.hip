@@ -815,10 +815,10 @@ int pick_splits(int64_t items, int64_t key_blocks, int cus) {
  * over 512 keys 11.2 -> 10.0; 512 heads, 16 queries over 100 6.3 -> 5.7),
  * where the keys would not be cut three ways or more (4 heads, 64 queries over
  * 4000 keys in 3 splits 23.7 against 32.5; 256 workgroups 37.4 -> 35.5).
- * Head size 128 (one to a CU): up to one round, and half of one where they are
- * not more than one group's and the keys few (64 queries a head over 512 keys,
- * 128 heads 14.8 -> 13.8, 256 heads 17.1 against 17.4, 33 over 1500 36.8 ->
- * 33.2), from 4 blocks of keys on (8 heads, 200 queries over 100 keys 6.9
+ * Head size 128 (one to a CU): up to one round, and two thirds of one where
+ * they are not more than one group's and the keys few (44 queries a head over
+ * 398 keys, 160 heads 13.1 -> 12.5, 192 heads 13.5 against 13.8; 256 heads, 33
+ * over 1500 36.8 -> 33.2), from 4 blocks of keys on (8 heads, 200 queries over 100 keys 6.9
  * against 7.6, 1000 over 256 9.9 -> 9.1), where the keys would not be cut (512
  * queries of 32 heads over 2048 keys in 2 splits 36.0 against 35.1, over 8192
  * in 4 splits 87 against 125). Undivided launches (`allow_split` false) are
@@ -833,7 +833,7 @@ bool two_groups(int head_dim, int64_t seq_q, int64_t items, int64_t items64, int
     return items64 <= 2 * cus && key_blocks >= (items64 <= cus || seq_q <= 32 ? 2 : 5) &&
            (splits < 3 || (splits == 3 && items64 > cus / 2));
   }
-  return items64 <= (items64 > items || key_blocks >= 16 ? cus : cus / 2) && key_blocks >= 4 &&
+  return items64 <= (items64 > items || key_blocks >= 16 ? cus : 2 * cus / 3) && key_blocks >= 4 &&
          splits == 1;
 }
 
