@@ -1,7 +1,8 @@
-"""The f32 GEMM on bf16 planes, and on f32 MFMAs (gemm_f32.hip): what its planes cannot hold,
-and the edges of its stages, against the f64 product. The tolerance is the
-bound of f32 sums of products in any order plus what the dropped planes'
-products come to: |C - AB| <= (K + 2) 2^-24 (|A| |B|)."""
+"""The f32 GEMM on bf16 planes, and on f32 MFMAs where K is short
+(gemm_f32.hip): what its planes cannot hold, and the edges of its stages,
+against the f64 product. The tolerance is the bound of f32 sums of products in
+any order plus what the planes' products left out come to, 2^-24 of each:
+|C - AB| <= (K + 2) 2^-24 (|A| |B|)."""
 
 import numpy as np
 import pytest

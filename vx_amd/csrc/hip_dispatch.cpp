@@ -439,7 +439,7 @@ void stage(const void *data, int64_t rows, int64_t cols, int64_t row_stride,
 }
 
 /* `no_alloc`: the no-alloc entry point's call, which takes no device memory
- * beyond its scratch (so no stream-K workspace either). */
+ * beyond its scratch (so no workspace either). */
 bool run_gemm(const vx_gemm_plan &plan, Arena *arena = nullptr, bool no_alloc = false) {
   const size_t in_esz = vx_dtype_bytes(plan.dtype);
   const size_t out_esz = vx_dtype_bytes(plan.out_dtype);
@@ -1537,11 +1537,10 @@ int64_t vx_plugin_tensor_map(int64_t base, int64_t rank, int64_t elem_bytes,
 /* The caller stream, as a hipStream_t. The CUDA-named pair is what compiled
  * programs and host code already call (reference
  * runtime/cuda_dispatch.cpp:2030-2035); the HIP-named pair is the same.
- * Moving off a stream frees, in that stream's order, the flash-attention
- * split workspace and the stream-K GEMM workspace the library kept for it,
- * so a stream the caller then
- * destroys leaves nothing behind and a later stream at the same address
- * starts with none. A stream must stay alive while it is set. */
+ * Moving off a stream frees, in that stream's order, the attention and GEMM
+ * workspaces the library kept for it, so a stream the caller then destroys
+ * leaves nothing behind and a later stream at the same address starts with
+ * none. A stream must stay alive while it is set. */
 void vx_hip_set_stream(void *stream) {
   const hipStream_t next = static_cast<hipStream_t>(stream);
   if (caller_stream && caller_stream != next) {

@@ -1089,8 +1089,8 @@ bool gemm_kernel_takes(GemmKernel which, const GemmArgs &g) {
 
 GemmKernel gemm_pick(const GemmArgs &g) {
   /* 16-bit products of 2^18 multiply-adds and K >= 128, of 2^25, or of 2^24
-   * where rows and K allow the tiles' loads: MFMA kernels (smaller ones stay exact-order: a launch is most of their time,
-   * 64^3 6.0 us). Of the register GEMM and, where rows and K allow their
+   * where rows and K allow the tiles' loads: MFMA kernels (smaller ones stay
+   * exact-order: a launch is most of their time, 64^3 6.0 us). Of the register GEMM and, where rows and K allow their
    * loads, 128x128 and 256x256 tiles, the one of least time by its model:
    * 512 x 4096 x 4096 34, 45 and 88 us, 1024 x 4096 x 4096 66, 49 and 90,
    * 4096^3 215, 148 and 113. Grids of more than one round of 256x256 tiles
@@ -1124,7 +1124,8 @@ GemmKernel gemm_pick(const GemmArgs &g) {
   /* f32: the exact-order kernel (bit-equal to the reference's host loop)
    * below 2^30 multiply-adds, the MFMA kernel above, also where most of its
    * tile is past the last row (10 x 12000 x 12000 553 -> 239 us, 100 x 4000 x
-   * 4000 188 -> 36). */
+   * 4000 188 -> 36), the last column (2^20 x 8 x 128 410 -> 314) or both (64 x
+   * 64 x 262144 5000 -> 590, 8 x 8 x 2^24 307 -> 36 ms). */
   if (g.m >= 8 && g.n >= 8 && (double)g.m * g.n * g.k >= 1073741824.0 &&
       f32_mfma_takes(g)) {
     return GEMM_F32_MFMA;

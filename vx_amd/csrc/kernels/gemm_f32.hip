@@ -35,11 +35,12 @@
  * bounds it. The planes' way there, against it: 8192^2 x 16 103 us, 52; 328 x
  * 601168 x 8 365, 197; 4096^2 x 64 34, 27.
  *
- * Against f32 MFMAs in the same tile: 2048^3 248 -> 92 us with new inputs each
- * pass (188 TFLOP/s), 258 -> 104 with the same ones; error against 64 bits
- * 8.1e-7 -> 2.5e-7 at 2048^3, 1.1e-6 -> 3.8e-7 at K = 4096. Grids of fewer
- * tiles than CUs divide K over workgroups: 1024^3 125 -> 27 us (undivided 45),
- * 128 x 4096 x 4096 454 -> 38 (142).
+ * Against f32 MFMAs in the same tile: 2048^3 248 -> 90 us with new inputs each
+ * pass (191 TFLOP/s); error against 64 bits 8.1e-7 -> 2.5e-7 at 2048^3, 1.1e-6
+ * -> 3.8e-7 at K = 4096. Watching the least magnitude is 3% of that (24 of a
+ * stage's 120 vector instructions a wave). Grids of fewer tiles than CUs divide
+ * K over workgroups: 1024^3 125 -> 25 us (undivided 45), 128 x 4096 x 4096 454
+ * -> 37 (142).
  */
 #include "../vx_hip_common.h"
 #include "../vx_kernels.h"

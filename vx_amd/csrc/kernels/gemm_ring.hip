@@ -13,9 +13,10 @@
  *
  * A stage takes 0.34 us where a CU has one workgroup and 0.53 where it has
  * two (690 TFLOP/s at 1024 x 4096 x 4096); what bounds it is getting 16 KiB a
- * stage and workgroup through L1 from L2 (the TCP waits 38% of the cycles,
- * the matrix cores work 41%, the LDS reads take a fifth); for 256x128, 24 KiB
- * and 0.47 us, or 0.57 with B from HBM. With four waves the larger tiles leave
+ * stage and workgroup through L1 from L2 (the TCP waits on L2 60% of its
+ * cycles, the matrix cores work 30% of a wave's time, no LDS read conflicts);
+ * for 256x128, 24 KiB and 0.47 us, or 0.57 with B from HBM (TCP 38%, matrix
+ * cores 44%). With four waves the larger tiles leave
  * the loads' latency open: 128x192 gave 67.5 us at 512 x 11008 x 4096 and 61 at
  * 1024 x 4096 x 4096 against 70.7 and 49, 256x128 78.8 and 70. Against the kernels
  * that took these shapes: 512 x 11008 x 4096 102 -> 76 us with

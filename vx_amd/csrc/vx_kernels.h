@@ -29,8 +29,8 @@ struct GemmArgs {
    * and real-time counter at the start and end of workgroup 0), or null. */
   uint64_t *stamp = nullptr;
   /* Whether the launch may take a workspace of its own (false under graph
-   * capture and for the no-alloc entry point): the stream-K launch and the
-   * register GEMM's splits need one. */
+   * capture, for the no-alloc entry point and under hipStreamPerThread): the
+   * stream-K launch and those that divide a tile's K need one. */
   bool may_split = false;
 };
 
@@ -64,8 +64,7 @@ bool gemm_launch(const GemmArgs &g, hipStream_t stream);
 bool gemm_launch_kernel(GemmKernel which, const GemmArgs &g,
                         hipStream_t stream);
 
-/* Frees, in `stream`'s order, the workspaces (stream-K, the register GEMM's
- * splits) kept for `stream` on every device (none while it is capturing); the
+/* Frees, in `stream`'s order, the workspaces (stream-K, divided K) kept for `stream` on every device (none while it is capturing); the
  * number freed. */
 int gemm_release_stream(hipStream_t stream);
 /* Workspaces held, their bytes, and stream-K launches so far. */

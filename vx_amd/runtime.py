@@ -140,7 +140,7 @@ class DispatchLibrary:
 
     def gemm_workspaces(self) -> dict:
         """GEMM workspaces held (one per device, stream and kind that ran there:
-        stream-K, the register GEMM's splits), their bytes, stream-K launches so far, and the
+        stream-K, divided K), their bytes, stream-K launches so far, and the
         workgroups (CUs) such a launch runs."""
         out = (ctypes.c_int64 * 4)()
         if not self.lib.vx_plugin_control(abi.HIP_CTRL_GEMM_WORKSPACES, out):
