@@ -13,7 +13,7 @@ namespace f32 {
 constexpr int kTile = 128;
 constexpr int kPart = kTile * kTile * 4; /* bytes of a split's sums of a tile */
 /* K from which the bf16 planes are taken: below it a tile is its loads, its
- * start and writing C, and f32 MFMAs do with a third of the LDS (planes and
+ * start and writing C, and f32 MFMAs do with a sixth of the LDS (planes and
  * f32: 4096^2 x 96 39.7 us and 36.0, x 128 44.1 and 43.6, x 160 49.3 and 51.7;
  * 3000^2 x 128 32.3 and 33.7; 2^20 x 8 x 128 314 and 290, x 192 411 and 421). */
 constexpr int64_t kPlanesMinK = 128;

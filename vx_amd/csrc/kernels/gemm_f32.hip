@@ -12,7 +12,7 @@
  *
  * What bf16 cannot hold is left to f32 MFMAs: a block of 16 x 16 sums is
  * computed again that way, over the workgroup's k, where one of them is not
- * finite or lies below 2^-100, or where an element below 2^-100 may have lost
+ * finite or lies below 2^-100 (but not 0), or where an element below 2^-100 may have lost
  * bits that count in it. The last needs, of each row and column, the greatest
  * magnitude and whether it has such an element; a tile that met one reads its
  * operands again for them (2048^3 with a third of A below 2^-110 124 us, with
@@ -30,10 +30,12 @@
  * barriers (taking a SIMD's two waves in turns, one reading while the other
  * multiplies, costs a barrier more and gave the same: 108 us).
  *
- * K below f32::kPlanesMinK: the same tile on f32 MFMAs throughout, one LDS slot
- * and three workgroups to a CU, whose loads and stores overlap. Writing C
- * bounds it. The planes' way there, against it: 8192^2 x 16 103 us, 52; 328 x
- * 601168 x 8 365, 197; 4096^2 x 64 34, 27.
+ * K below f32::kPlanesMinK: the same tile on f32 MFMAs throughout, stages of 16
+ * through one LDS slot and three workgroups to a CU, whose loads and stores
+ * overlap. Writing C bounds it. The planes' way there, against it: 8192^2 x 16
+ * 103 us, 47; 64280 x 2576 x 18 247, 148; 4096^2 x 64 34, 30; 8 x 8388608 x 16
+ * 1195, 500. (Stages of 32: 52, 168, 29 and 590; four workgroups to a CU spill:
+ * 49, 162, 29 and 482.)
  *
  * Against f32 MFMAs in the same tile: 2048^3 248 -> 90 us with new inputs each
  * pass (191 TFLOP/s); error against 64 bits 8.1e-7 -> 2.5e-7 at 2048^3, 1.1e-6
@@ -55,9 +57,7 @@ namespace {
 
 constexpr int kThreads = 512;
 constexpr int kTile = f32::kTile;
-constexpr int kKs = 32;               /* of k per stage */
 constexpr int kPlane = kTile * 4;     /* 16-byte units */
-constexpr int kRows32 = kTile * 8;    /* of a stage's rows in f32 */
 constexpr float kLeast = 7.888609052210118e-31f; /* 2^-100 */
 constexpr uint32_t kLeastBits = (127 - 100) << 23;
 
@@ -65,13 +65,16 @@ struct __attribute__((packed, aligned(4))) Four {
   f32x4 v;
 };
 
-struct Regs {
-  float a[8], b[8];
+/* A thread's k of a stage: of one row of A and of one column of B. */
+template <int kPer> struct Regs {
+  float a[kPer], b[kPer];
 };
 
 __device__ __forceinline__ int unit(int row, int c) { return row * 4 + (c ^ ((row >> 1) & 3)); }
-/* The same in f32, a chunk being 4 k. */
-__device__ __forceinline__ int unit32(int row, int c) { return row * 8 + (c ^ (row & 7)); }
+/* The same in f32, a chunk being 4 k, kC of them a row. */
+template <int kC> __device__ __forceinline__ int unit32(int row, int c) {
+  return kC == 4 ? unit(row, c) : row * kC + (c ^ (row & (kC - 1)));
+}
 
 /* Two values rounded to bf16, the first in the lower half. */
 __device__ __forceinline__ uint32_t round2(float lo, float hi) {
@@ -96,10 +99,15 @@ __device__ __forceinline__ void split8(const float (&x)[8], u32x4 (&p)[3]) {
 }
 
 template <bool kPlanes>
-__global__ __launch_bounds__(kThreads, kPlanes ? 2 : 6) void gemm_f32_mfma(
+__global__ __launch_bounds__(kThreads, kPlanes ? 2 : 7) void gemm_f32_mfma(
     const float *__restrict__ A, const float *__restrict__ B, float *__restrict__ C, int64_t M,
     int64_t N, int64_t K, int64_t lda, int64_t ldb, int64_t ldc, int tiles_m, int tiles_n,
     int splits, char *__restrict__ ws) {
+  constexpr int kPer = kPlanes ? 8 : 4;  /* of k per thread and stage */
+  constexpr int kKs = 4 * kPer;
+  constexpr int kC = kKs / 4;            /* chunks of a row in f32 */
+  constexpr int kRows32 = kTile * kC;    /* 16-byte units of a stage's rows in f32 */
+  using Regs = vxk::Regs<kPer>;
   /* [slot][A, B][plane][kPlane]; in f32 [slot][A, B][kRows32], one slot alone */
   __shared__ u32x4 lds[kPlanes ? 2 * 2 * 3 * kPlane : 2 * kRows32];
   const int t = threadIdx.x;
@@ -126,15 +134,15 @@ __global__ __launch_bounds__(kThreads, kPlanes ? 2 : 6) void gemm_f32_mfma(
   const int64_t stages = all * (split + 1) / splits - first;
   const int64_t whole = min(first + stages, K / kKs) - first;
   const int64_t left = K - first * kKs; /* k from its first on */
-  const float *pa = A + min(m0 + a_row, M - 1) * lda + first * kKs + 8 * a_chunk;
+  const float *pa = A + min(m0 + a_row, M - 1) * lda + first * kKs + kPer * a_chunk;
   const int b_off = (int)(min(n0 + b_col, N - 1) - n0);
-  const float *pb = B + (first * kKs + 8 * b_chunk) * ldb + n0;
+  const float *pb = B + (first * kKs + kPer * b_chunk) * ldb + n0;
 
   auto load = [&](Regs &r, int64_t st) {
     const float *a = pa + st * kKs;
     const float *b = pb + st * kKs * ldb;
 #pragma unroll
-    for (int h = 0; h < 2; ++h) {
+    for (int h = 0; h < kPer / 4; ++h) {
       const f32x4 v = reinterpret_cast<const Four *>(a)[h].v;
 #pragma unroll
       for (int e = 0; e < 4; ++e) {
@@ -142,7 +150,7 @@ __global__ __launch_bounds__(kThreads, kPlanes ? 2 : 6) void gemm_f32_mfma(
       }
     }
 #pragma unroll
-    for (int e = 0; e < 8; ++e) {
+    for (int e = 0; e < kPer; ++e) {
       r.b[e] = (b + e * ldb)[b_off];
     }
   };
@@ -150,9 +158,9 @@ __global__ __launch_bounds__(kThreads, kPlanes ? 2 : 6) void gemm_f32_mfma(
     const float *a = pa + st * kKs;
     const float *b = pb + st * kKs * ldb;
 #pragma unroll
-    for (int e = 0; e < 8; ++e) {
-      r.a[e] = st * kKs + 8 * a_chunk + e < left ? a[e] : 0.0f;
-      r.b[e] = st * kKs + 8 * b_chunk + e < left ? (b + e * ldb)[b_off] : 0.0f;
+    for (int e = 0; e < kPer; ++e) {
+      r.a[e] = st * kKs + kPer * a_chunk + e < left ? a[e] : 0.0f;
+      r.b[e] = st * kKs + kPer * b_chunk + e < left ? (b + e * ldb)[b_off] : 0.0f;
     }
   };
   auto load_any = [&](Regs &r, int64_t st) {
@@ -172,10 +180,10 @@ __global__ __launch_bounds__(kThreads, kPlanes ? 2 : 6) void gemm_f32_mfma(
   auto in_f32 = [&](uint32_t blocks) {
     auto stash = [&](const Regs &r, int slot) {
 #pragma unroll
-      for (int h = 0; h < 2; ++h) {
-        lds[2 * slot * kRows32 + unit32(a_row, 2 * a_chunk + h)] = __builtin_bit_cast(
+      for (int h = 0; h < kPer / 4; ++h) {
+        lds[2 * slot * kRows32 + unit32<kC>(a_row, kPer / 4 * a_chunk + h)] = __builtin_bit_cast(
             u32x4, f32x4{r.a[4 * h], r.a[4 * h + 1], r.a[4 * h + 2], r.a[4 * h + 3]});
-        lds[(2 * slot + 1) * kRows32 + unit32(b_col, 2 * b_chunk + h)] = __builtin_bit_cast(
+        lds[(2 * slot + 1) * kRows32 + unit32<kC>(b_col, kPer / 4 * b_chunk + h)] = __builtin_bit_cast(
             u32x4, f32x4{r.b[4 * h], r.b[4 * h + 1], r.b[4 * h + 2], r.b[4 * h + 3]});
       }
     };
@@ -211,18 +219,18 @@ __global__ __launch_bounds__(kThreads, kPlanes ? 2 : 6) void gemm_f32_mfma(
         lds_barrier();
       }
 #pragma unroll
-      for (int h = 0; h < 2; ++h) {
+      for (int h = 0; h < kC / 4; ++h) {
         if (st * kKs + 16 * h < left) {
           f32x4 af[4], bf[2];
 #pragma unroll
           for (int i = 0; i < 4; ++i) {
             af[i] = __builtin_bit_cast(
-                f32x4, lds[2 * slot * kRows32 + unit32(64 * wm + 16 * i + l16, 4 * h + g)]);
+                f32x4, lds[2 * slot * kRows32 + unit32<kC>(64 * wm + 16 * i + l16, 4 * h + g)]);
           }
 #pragma unroll
           for (int j = 0; j < 2; ++j) {
             bf[j] = __builtin_bit_cast(
-                f32x4, lds[(2 * slot + 1) * kRows32 + unit32(32 * wn + 16 * j + l16, 4 * h + g)]);
+                f32x4, lds[(2 * slot + 1) * kRows32 + unit32<kC>(32 * wn + 16 * j + l16, 4 * h + g)]);
           }
 #pragma unroll
           for (int i = 0; i < 4; ++i) {
