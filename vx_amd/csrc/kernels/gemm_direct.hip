@@ -82,9 +82,9 @@ template <int kOut> __device__ __forceinline__ void put8(char *c, int64_t at, co
   }
 }
 
-template <bool kBf16, int kOut, int kMT, int kBuf, bool kAlongK, bool kOddA>
+template <bool kBf16, int kOut, int kMT, int kBuf, bool kAlongK, bool kOddA, bool kStamp>
 __global__ __launch_bounds__(kThreads, kMT <= 2 ? 2 : 1) void gemm_direct(DirectArgs p) {
-  const ClockStamp clocks(p.stamp);
+  const ClockStamp<kStamp> clocks(p.stamp);
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int l16 = lane & 15;
@@ -385,14 +385,12 @@ __global__ __launch_bounds__(kThreads, kMT <= 2 ? 2 : 1) void gemm_direct(Direct
  * 4096 x 4096 11.4 and 12.2, 1000 x 777 x 1111 13.1 and 12.9). */
 template <bool kBf16, int kOut, int kMT, int kBuf, int kBufOdd, bool kAlongK>
 void launch(const DirectArgs &p, hipStream_t s) {
-  const dim3 grid(p.tiles_m * p.tiles_n * p.splits);
-  if ((p.lda & 1) || (reinterpret_cast<uintptr_t>(p.a) & 2)) {
-    hipLaunchKernelGGL((gemm_direct<kBf16, kOut, kMT, kBufOdd, kAlongK, true>), grid,
-                       dim3(kThreads), 0, s, p);
-  } else {
-    hipLaunchKernelGGL((gemm_direct<kBf16, kOut, kMT, kBuf, kAlongK, false>), grid,
-                       dim3(kThreads), 0, s, p);
-  }
+  const bool odd = (p.lda & 1) || (reinterpret_cast<uintptr_t>(p.a) & 2);
+  const auto kernel = odd ? p.stamp ? gemm_direct<kBf16, kOut, kMT, kBufOdd, kAlongK, true, true>
+                                    : gemm_direct<kBf16, kOut, kMT, kBufOdd, kAlongK, true, false>
+                      : p.stamp ? gemm_direct<kBf16, kOut, kMT, kBuf, kAlongK, false, true>
+                                : gemm_direct<kBf16, kOut, kMT, kBuf, kAlongK, false, false>;
+  hipLaunchKernelGGL(kernel, dim3(p.tiles_m * p.tiles_n * p.splits), dim3(kThreads), 0, s, p);
 }
 
 template <bool kBf16, int kOut>

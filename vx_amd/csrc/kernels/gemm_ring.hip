@@ -71,12 +71,12 @@ template <int kOut> __device__ __forceinline__ void put4(void *c, int64_t at, f3
   }
 }
 
-template <bool kBf16, int kOut, int kBM>
+template <bool kBf16, int kOut, int kBM, bool kStamp>
 __global__ __launch_bounds__(2 * kBM, 2) void gemm_ring(
     const uint16_t *__restrict__ A, const uint16_t *__restrict__ B, void *__restrict__ C,
     int64_t M, int64_t N, int K, int64_t lda, int64_t ldb, int64_t ldc, int tiles_m,
     int tiles_n, int splits, char *__restrict__ ws, uint64_t *__restrict__ stamp) {
-  const ClockStamp clocks(stamp);
+  const ClockStamp<kStamp> clocks(stamp);
   constexpr int kThreads = 2 * kBM;                         /* a wave per 64x64 */
   constexpr int kNS = kBM == 128 ? 5 : 6;                   /* slots: 80 KiB, or 144 */
   constexpr int kUA = kBM * 4;                              /* 16-byte units per stage */
@@ -287,8 +287,9 @@ __global__ __launch_bounds__(2 * kBM, 2) void gemm_ring(
 template <bool kBf16, int kOut, int kBM>
 void launch_rows(const GemmArgs &g, int splits, char *ws, hipStream_t s) {
   const int tiles_m = (int)((g.m + kBM - 1) / kBM), tiles_n = (int)((g.n + kBN - 1) / kBN);
-  hipLaunchKernelGGL((gemm_ring<kBf16, kOut, kBM>), dim3(tiles_m * tiles_n * splits),
-                     dim3(2 * kBM), 0, s, static_cast<const uint16_t *>(g.a), static_cast<const uint16_t *>(g.b),
+  const auto kernel = g.stamp ? gemm_ring<kBf16, kOut, kBM, true> : gemm_ring<kBf16, kOut, kBM, false>;
+  hipLaunchKernelGGL(kernel, dim3(tiles_m * tiles_n * splits), dim3(2 * kBM), 0, s,
+                     static_cast<const uint16_t *>(g.a), static_cast<const uint16_t *>(g.b),
                      g.c, g.m, g.n, (int)g.k, g.lda, g.ldb, g.ldc, tiles_m, tiles_n, splits, ws,
                      g.stamp);
 }
